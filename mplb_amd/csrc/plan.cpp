@@ -268,6 +268,36 @@ int Plan::region_of(int b, int i, int j, int k) const {
     return r;
 }
 
+// the wall-velocity terms of KerCutCellEQMDiffuseRefl[3D] (boundary_kernel.
+// inc:534-613, 1184-1276) in precision T, in the reference's order
+template <typename T>
+static void eqm_terms(const BCOp& op, const LatticeTab& L, T* den, T* cq) {
+    const T cs = T(std::sqrt(3.0));
+    const T u = T(op.vars[0]), v = T(op.vars[1]), w = T(op.vars[2]);
+    const bool d3 = L.Q > 9;
+    T drho = T(0), rpar = T(0);
+    for (int q = 0; q < L.Q; q++) {
+        T cu = cs * T(L.C[q][0]) * u + cs * T(L.C[q][1]) * v;
+        T u2 = u * u + v * v;
+        if (d3) {
+            cu = cu + cs * T(L.C[q][2]) * w;
+            u2 = u2 + w * w;
+        }
+        const T wq = T(L.W[q]);
+        cq[q] = T(0);
+        if (op.m_in >> q & 1u) continue;
+        if (op.m_out >> q & 1u) {
+            drho += (T(2) * wq) * cu;
+            cq[q] = T(2) * cu;
+        } else if (op.m_par >> q & 1u) {
+            const T res = T(1.0) + cu + T(0.5) * (cu * cu - u2);
+            rpar += wq * T(1) * res;
+            cq[q] = res;
+        }
+    }
+    *den = T(1) - drho - rpar;
+}
+
 static void region_rep(int dim, const int n[3], int r, int p[3]) {
     int code[3] = {r % 3, (r / 3) % 3, r / 9};
     for (int a = 0; a < 3; a++) {
@@ -524,6 +554,33 @@ bool Plan::build() {
         error = "persisted boundary state too large";
         return false;
     }
+    // A wall application reads only the incoming populations and writes every
+    // other class, the classes being the region's: of several on one region
+    // (edges and corners, where the last-defined boundary wins) only the last
+    // leaves a trace.  Regions whose sequence an extrapolation reads part way
+    // keep theirs.
+    std::vector<char> read((size_t)nb * nregions, 0);
+    for (int b = 0; b < nb; b++)
+        for (int r = 0; r < nregions; r++) {
+            const RegionProg& P = progs[(size_t)b * nregions + r];
+            for (int o = 0; o < P.nops; o++)
+                if (P.op[o].type == OP_EXTRAPOL && P.op[o].m_ext)
+                    read[(size_t)b * nregions + P.op[o].nb_region] = 1;
+        }
+    for (size_t i = 0; i < progs.size(); i++) {
+        RegionProg& P = progs[i];
+        bool walls = P.nops > 1 && !read[i];
+        for (int o = 0; o < P.nops; o++) {
+            const BCOp &a = P.op[o], &l = P.op[P.nops - 1];
+            walls = walls && a.type == OP_EQM && a.m_in == l.m_in && a.m_out == l.m_out &&
+                    a.m_par == l.m_par && (l.m_in & (l.m_out | l.m_par)) == 0;
+            for (int q = 0; q < Q; q++)
+                if (l.m_out >> q & 1u) walls = walls && (l.m_in >> OPP[q] & 1u);
+        }
+        if (!walls) continue;
+        P.op[0] = P.op[P.nops - 1];
+        P.nops = 1;
+    }
     const double cs = std::sqrt(3.0);
     for (int b = 0; b < nb; b++)
         for (int r = 0; r < nregions; r++) {
@@ -551,6 +608,8 @@ bool Plan::build() {
                         op.eq_c[q] = (float)f1;
                     }
                 }
+                eqm_terms(op, L, &op.den, op.cq);
+                eqm_terms(op, L, &op.fden, op.fcq);
                 op.eq_win = (float)win;
                 op.eq_k = (float)(2.0 / (1.0 - drho - rpar));
             }

@@ -62,6 +62,11 @@ struct BCOp {
     float eq_win;                 // sum of w over m_in
     float eq_k;                   // 2 / (1 - dRho - rhoPar)
     float eq_c[kMaxQ];            // parallel: w res(u); outgoing: 2 w c.u
+    // the same on full values, each term with the kernel's roundings in FP64
+    // and in FP32: rho_w = 2 sum_in f / den; cq = res(u) (parallel),
+    // 2 CS c.u (outgoing) or 0
+    double den, cq[kMaxQ];
+    float fden, fcq[kMaxQ];
 };
 
 struct RegionProg {
