@@ -588,9 +588,10 @@ def main():
                      "boundary_kernel_avg_ms": round(ms_bnd / K, 5),
                      "step_kernels_avg_ms": round(ms_kernel / K, 5),
                      "ms_per_step_event_timed": round(wall_events / K * 1e3, 5),
-                     "timing": "value: K steps of graph replays (the production path); "
-                               "kernel times: HIP events around every kernel of K more "
-                               "steps launched one by one on the same streams",
+                     "timing": "value: K steps of the production path (two steps per launch, "
+                               "k_pair, in graph replays); this roofline: the single-step "
+                               "kernels, HIP events around every kernel of K more steps "
+                               "launched one by one on the same streams",
                      "copy_probe_GBs": round(copy_gbs, 1),
                      "frac_of_copy": round(achieved / copy_gbs, 4)},
         "cpu_baseline": cpu,

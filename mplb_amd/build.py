@@ -16,7 +16,8 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
-SOURCES = ["plan.cpp", "mplbhip.cpp", "lattice_kernels.hip", "swap_kernels.hip"]
+SOURCES = ["plan.cpp", "mplbhip.cpp", "lattice_kernels.hip", "pair_kernels.hip",
+           "swap_kernels.hip"]
 
 
 WS_OUT = os.path.join(HERE, "libmplbws.so")
@@ -31,7 +32,7 @@ def build(verbose=False):
 
 def _build_lib(sources, target, verbose):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    objs = []
+    objs, jobs = [], []
     os.makedirs(os.path.join(HERE, "_build"), exist_ok=True)
     for src in sources:
         obj = os.path.join(HERE, "_build", os.path.splitext(src)[0] + ".o")
@@ -40,8 +41,11 @@ def _build_lib(sources, target, verbose):
             cmd[1:1] = ["-x", "hip"]
         if verbose:
             print(" ".join(cmd), flush=True)
-        subprocess.check_call(cmd)
+        jobs.append((cmd, subprocess.Popen(cmd)))
         objs.append(obj)
+    for cmd, job in jobs:
+        if job.wait() != 0:
+            raise subprocess.CalledProcessError(job.returncode, cmd)
     tmp = target + ".tmp"
     cmd = [hipcc, "--offload-arch=" + ARCH, "-shared", "-o", tmp] + objs
     subprocess.check_call(cmd)

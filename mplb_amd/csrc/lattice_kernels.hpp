@@ -120,6 +120,19 @@ enum Mode : int {
     MODE_INIT_F = 4       // f from host-layout array -> collide -> fs_next
 };
 
+// Two steps in one launch (k_pair): the tiling of one block.  A workgroup
+// owns w x h columns of one range of lz z planes and marches through them;
+// it computes the first of the two steps on its tile plus one node on every
+// side.  nt: threads of the workgroup, at least (w + 2)(h + 2).
+struct PairBlock {
+    int32_t start;       // first workgroup of this block
+    int32_t w, h, lz;
+    int32_t tx, ty, tz;  // tiles along each axis
+    // tx and ty as multiply-high-and-shift divisors
+    uint32_t div_m[2];
+    int32_t div_sh[2];
+};
+
 struct KParams {
     const BlockParams* blocks;
     int32_t nblocks;
@@ -172,6 +185,12 @@ struct KParams {
     const int32_t* wg_block_bulk3;
     const int32_t* wg_block_h2;
     const int32_t* wg_block_bnd;
+    // two-step launches: each block's tiling, the block of every workgroup,
+    // the workgroups and their threads
+    const PairBlock* pair;
+    const int32_t* wg_block_pair;
+    int32_t npair;
+    int32_t pair_nt;
 };
 
 struct HaloParams {

@@ -23,6 +23,8 @@ namespace mplbhip {
 hipError_t launch_lattice(int dim, int storage, int mode, const KParams& kp,
                           hipStream_t s, int part = 0);
 hipError_t launch_materialize_split(int dim, int storage, const KParams& kp, hipStream_t s);
+bool pair_shape(int storage, int nt, int* positions);
+hipError_t launch_pair(int lat, int storage, const KParams& kp, hipStream_t s);
 hipError_t launch_halo(const HaloParams& hp, hipStream_t s);
 hipError_t launch_halo_multi(const HaloParams* links, const int32_t* wg_start, int nlinks,
                              int nwg, int Q, int elem_bytes, hipStream_t s);
@@ -124,6 +126,16 @@ struct mplbhip_ctx {
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     bool fold_env = false, xgroup_env = false;  // fixed by the environment
+    // two steps per launch (k_pair): allowed by the case (1 forced, -1
+    // forbidden by MPLBHIP_PAIR), in use over the blocks the launches cover,
+    // each block's tiling, and the block of every workgroup
+    bool pair_ok = false, pair = false;
+    int pair_env = 0;
+    std::vector<PairBlock> pb;
+    std::vector<int32_t> wg_pair_host;
+    int npair = 0, pair_nt = 0;
+    DevBuf dpair, wg_pair;
+    int singles = 0;  // single steps taken before their launch was tuned
     std::vector<BndSeg> segs;
     std::vector<std::vector<uint8_t>> solid;  // obstacle nodes per block (empty: none)
     std::vector<uint32_t> obst;               // link masks per interior node
@@ -307,6 +319,10 @@ static KParams base_params(mplbhip_ctx* c) {
         kp.wg_block_h2 = wgb + c->wg_block_off[kWgH2];
         kp.wg_block_bnd = wgb + c->wg_block_off[kWgBnd + fold];
     }
+    kp.pair = static_cast<const PairBlock*>(c->dpair.p);
+    kp.wg_block_pair = static_cast<const int32_t*>(c->wg_pair.p);
+    kp.npair = c->npair;
+    kp.pair_nt = c->pair_nt;
     return kp;
 }
 
@@ -414,6 +430,19 @@ static int enqueue_step(mplbhip_ctx* c, bool check, bool residual) {
     return 0;
 }
 
+// two steps in one launch from parity c->cur; leaves c->cur flipped.  The
+// other fStage buffer then holds the state two steps back, so a run whose
+// result is measured by re-streaming ends with a single step.
+static int enqueue_pair(mplbhip_ctx* c) {
+    HIPCHK(c, launch_pair(c->lat, c->storage, base_params(c), c->stream));
+    c->cur ^= 1;
+    return 0;
+}
+
+// two-step launches in force: a body force given after prepare turns them off
+static bool use_pair(const mplbhip_ctx* c) {
+    return c->pair && !c->force_type && !c->force_macros;
+}
 
 static int build_graphs(mplbhip_ctx* c, int nsteps) {
     drop_graphs(c);
@@ -422,7 +451,10 @@ static int build_graphs(mplbhip_ctx* c, int nsteps) {
         const int saved = c->cur;
         c->cur = p;
         int rc = 0;
-        for (int s = 0; s < nsteps && rc == 0; s++) rc = enqueue_step(c, false, false);
+        if (use_pair(c))
+            for (int s = 0; s < nsteps && rc == 0; s += 2) rc = enqueue_pair(c);
+        else
+            for (int s = 0; s < nsteps && rc == 0; s++) rc = enqueue_step(c, false, false);
         c->cur = saved;
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(c->stream, &g);
@@ -1288,6 +1320,134 @@ static int assign_tiles(mplbhip_ctx* c, bool only_active) {
     return grouped;
 }
 
+// Whether the case can take two steps per launch: 3D blocks without
+// connections or obstacles, BGK without a body force, every envelope region a
+// wall (masked pulls and at most one EQM application), populations persisted
+// at single corner nodes only, and rows long enough to tile.
+static bool pair_allowed(const mplbhip_ctx* c) {
+    if (c->dim != 3 || c->swap || c->thermal) return false;
+    if (!c->plan.links.empty() || !c->obst.empty()) return false;
+    for (size_t b = 0; b < c->plan.blocks.size(); b++) {
+        if (c->bp[b].n[0] < 16 || c->bp[b].n[1] < 4) return false;
+        for (int r = 1; r < c->plan.nregions; r++) {
+            const RegionProg& P = c->plan.progs[b * c->plan.nregions + r];
+            const bool corner = r % 3 && (r / 3) % 3 && r / 9;
+            if (P.kind != RK_MASKED || P.nops > 1) return false;
+            if (P.nops == 1 && P.op[0].type != OP_EQM) return false;
+            if (P.persist >= 0 && !corner) return false;
+        }
+    }
+    return true;
+}
+
+// Whether every tile of a w x h tiling of a block fits a k_pair workgroup of
+// nt threads and np positions: the grown tile's positions, and for either
+// step the threads of its nodes (the first wave for the x-face nodes).
+static bool pair_fits(const int* n, int w, int h, int nt, int np) {
+    if ((w + 2) * (h + 2) > np) return false;
+    for (int xa = 0; xa < n[0]; xa += w) {
+        const bool lo1 = xa <= 1, hi1 = xa + w + 1 >= n[0];
+        const bool lo = xa == 0, hi = xa + w >= n[0];
+        const int rw1 = (hi1 ? n[0] - 1 : xa + w + 1) - (lo1 ? 1 : xa - 1);
+        const int rows1 = std::min(h + 2, n[1]), rows = std::min(h, n[1]);
+        if ((lo1 || hi1 ? 64 : 0) + rw1 * rows1 > nt) return false;
+        if ((lo || hi ? 64 : 0) + w * rows > nt) return false;
+        if (rows1 * ((lo1 ? 1 : 0) + (hi1 ? 1 : 0)) > 64) return false;
+    }
+    return true;
+}
+
+static int upload_pairs(mplbhip_ctx* c) {
+    if (int rc = dalloc(c, c->dpair, c->pb.size() * sizeof(PairBlock))) return rc;
+    if (int rc = dalloc(c, c->wg_pair, std::max<size_t>(1, c->wg_pair_host.size()) * sizeof(int32_t)))
+        return rc;
+    HIPCHK(c, hipMemcpyAsync(c->dpair.p, c->pb.data(), c->dpair.bytes, hipMemcpyHostToDevice,
+                             c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->wg_pair.p, c->wg_pair_host.data(),
+                             c->wg_pair_host.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                             c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+}
+
+// The two-step tiling of one of nblk blocks, by a model of the launch: its
+// workgroups run in rounds of one per CU, each for lz + 3 planes (the planes
+// below and above its range, and the start); a plane costs a fixed latency,
+// worth that of 16 waves, and the work of the tile's waves, and the two ends
+// of its rows add a quarter of a 128-byte line.  Fitted to some 700 tilings
+// of 48^3 to 256^3 in the three storage forms, where its pick is within 8% of
+// the fastest.  Tile widths are multiples of 64 bytes (or the whole row):
+// rows that share such a piece with the next tile's cost twice the time
+// (D3Q19 FP32 256^3: 0.70 ms per step in tiles of 43 x 19, 0.28 in 64 x 13;
+// FP64 160^3: 0.27 in 20 x 18, 0.16 in 32 x 11).
+static void pair_tiling(const int* n, int es, long long nblk, int nt, int np, PairBlock* P) {
+    double best = 1e300;
+    const int unit = 64 / es;
+    for (int w = unit; w < n[0] + unit; w += unit) {
+        const int wt = w < n[0] ? w : n[0];
+        for (int ty = 1; ty <= n[1]; ty++) {
+            const int h = (n[1] + ty - 1) / ty;
+            if (!pair_fits(n, wt, h, nt, np)) continue;
+            const int waves = ((wt + 2) * (h + 2) + 63) / 64;
+            const long long columns = nblk * ((n[0] + wt - 1) / wt) * ((n[1] + h - 1) / h);
+            for (int tz = 1; tz <= n[2]; tz++) {
+                const int lz = (n[2] + tz - 1) / tz;
+                const long long wgs = columns * ((n[2] + lz - 1) / lz);
+                const double cost = (double)((wgs + 255) / 256) * (lz + 3) * (16.0 + waves) *
+                                    (1.0 + 32.0 / (wt * es));
+                if (cost < best) {
+                    best = cost;
+                    P->w = wt;
+                    P->h = h;
+                    P->lz = lz;
+                }
+            }
+            if (h < 4) break;
+        }
+    }
+}
+
+// Two-step launches over the (active) blocks: from 2^16 nodes on.  Below, a
+// step is bound by the launch and its latency either way (32^3 FP64: 11.1 us
+// per step against 9.8 in one whole-lattice launch; 48^3: 14.0 against 21.8).
+static int assign_pairs(mplbhip_ctx* c, bool only_active) {
+    c->pair = c->pair_ok && c->pair_env >= 0 && (c->pair_env > 0 || c->grid_nodes >= (1 << 16));
+    if (!c->pair) return 0;
+    int np = 0;
+    c->pair_nt = c->storage == MPLBHIP_STORE_F64 ? 512 : 1024;
+    if (!pair_shape(c->storage, c->pair_nt, &np))
+        return fail(c, MPLBHIP_ERR_HIP, "no two-step kernel for this storage");
+    long long nblk = 0;
+    for (const BlockParams& B : c->bp) nblk += !only_active || B.active ? 1 : 0;
+    c->pb.assign(c->bp.size(), PairBlock{});
+    c->wg_pair_host.clear();
+    for (size_t b = 0; b < c->bp.size(); b++) {
+        const BlockParams& B = c->bp[b];
+        PairBlock& P = c->pb[b];
+        P.start = (int32_t)c->wg_pair_host.size();
+        if (only_active && !B.active) continue;
+        if (b > 0 && std::equal(B.n, B.n + 3, c->bp[b - 1].n) && c->pb[b - 1].w > 0) {
+            P.w = c->pb[b - 1].w;
+            P.h = c->pb[b - 1].h;
+            P.lz = c->pb[b - 1].lz;
+        } else {
+            pair_tiling(B.n, (int)c->es, nblk, c->pair_nt, np, &P);
+        }
+        if (P.w <= 0) {  // no tile fits
+            c->pair = false;
+            return 0;
+        }
+        P.tx = (B.n[0] + P.w - 1) / P.w;
+        P.ty = (B.n[1] + P.h - 1) / P.h;
+        P.tz = (B.n[2] + P.lz - 1) / P.lz;
+        fast_div_params(P.tx, &P.div_m[0], &P.div_sh[0]);
+        fast_div_params(P.ty, &P.div_m[1], &P.div_sh[1]);
+        c->wg_pair_host.insert(c->wg_pair_host.end(), (size_t)P.tx * P.ty * P.tz, (int32_t)b);
+    }
+    c->npair = (int)c->wg_pair_host.size();
+    return upload_pairs(c);
+}
+
 // the workgroup -> block tables to the device (after assign_tiles; the
 // buffer holds the tables over every block, compaction only shrinks them)
 static int upload_wg_blocks(mplbhip_ctx* c) {
@@ -1512,6 +1672,11 @@ int mplbhip_prepare(mplbhip_ctx* c) {
     }
     if (int rc = upload_blocks(c)) return rc;
     if (int rc = upload_merged_halos(c)) return rc;
+    // a single-step form chosen by the environment is the one that runs
+    c->pair_ok = pair_allowed(c);
+    c->pair_env = c->fused_env || c->fold_env || c->xgroup_env || c->h2_env || c->xcd_remap ? -1 : 0;
+    if (const char* e = std::getenv("MPLBHIP_PAIR")) c->pair_env = std::atoi(e) != 0 ? 1 : -1;
+    if (int rc = assign_pairs(c, false)) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -1773,7 +1938,8 @@ static int first_collision(mplbhip_ctx* c) {
     }
     HIPCHK(c, launch_lattice(c->lat, c->storage, mode, kp, c->stream));
     if (int rc = exchange(c, 0)) return rc;
-    return autotune(c);
+    // with two-step launches the single ones only end a run: not tuned yet
+    return use_pair(c) ? 0 : autotune(c);
 }
 
 static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
@@ -1786,6 +1952,7 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         if (int rc = first_collision(c)) return rc;
     double ktot = 0.0;
     if (timed) {
+        if (int rc = autotune(c)) return rc;
         // per-step events bracket the bulk kernel and the boundary kernel,
         // each on the stream it runs on (the step's own launch structure)
         std::vector<hipEvent_t> evs(4 * (size_t)nsteps);
@@ -1846,17 +2013,29 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         if (g >= 2 && g <= 1024 && g % 2 == 0) G = g;
     }
     int left = nsteps;
-    if (left >= G) {
+    // two-step launches leave the last step to a single one
+    const bool pair = use_pair(c);
+    const int keep = pair ? 1 : 0;
+    if (left - keep >= G) {
         if (c->graph_steps != G)
             if (int rc = build_graphs(c, G)) return rc;
-        while (left >= G) {
+        while (left - keep >= G) {
             HIPCHK(c, hipGraphLaunch(c->gexec[c->cur], c->stream));
-            // G is even: the parity after G steps is unchanged
+            // G is even: single steps leave the parity unchanged
+            if (pair && (G / 2) % 2) c->cur ^= 1;
             c->tstep += G;
             left -= G;
         }
     }
+    while (pair && left - keep >= 2) {
+        if (int rc = enqueue_pair(c)) return rc;
+        c->tstep += 2;
+        left -= 2;
+    }
     while (left > 0) {
+        // a program that takes its steps one at a time gets them tuned too
+        if (pair && !c->tuned && ++c->singles > 64)
+            if (int rc = autotune(c)) return rc;
         if (int rc = enqueue_step(c, false, false)) return rc;
         c->tstep++;
         left--;
@@ -1950,7 +2129,7 @@ static int compact_grid(mplbhip_ctx* c, bool on) {
     c->fused = c->fused_env ? c->fused_full
                             : (on ? c->grid_nodes < (1 << 18) : c->fused_full);
     drop_graphs(c);
-    return 0;
+    return assign_pairs(c, on);
 }
 
 // Restart the listed blocks at rest, as a rest start forms its first
