@@ -223,6 +223,100 @@ __device__ __forceinline__ void apply_eqm_dev(float* g, const OP& op) {
     }
 }
 
+// FindBdyDvType[3D] (boundary_host_device.h:47-183, 191-706) of a face or an
+// edge region (2D: a corner): 1 streams into the wall, 2 comes out of it, 3 along it
+__host__ __device__ constexpr int wall_class(int D, int r, int q) {
+    const int code[3] = {r % 3, r / 3 % 3, r / 9};
+    int n = 0, cn[3] = {0, 0, 0};
+    for (int a = 0; a < 3; a++)
+        if (code[a]) cn[n++] = (code[a] == 1 ? 1 : -1) * cvel(D, q, a);
+    if (n == 1) return cn[0] < 0 ? 1 : cn[0] > 0 ? 2 : 3;
+    if ((cn[0] <= 0 && cn[1] < 0) || (cn[0] < 0 && cn[1] == 0)) return 1;
+    if ((cn[0] >= 0 && cn[1] > 0) || (cn[0] > 0 && cn[1] == 0)) return 2;
+    return 3;
+}
+
+// apply_eqm (DEV: apply_eqm_dev, on deviations) of region R with its
+// populations' classes known at compile time: every incoming population is
+// pulled, and every other one is written.  Reduced storage takes and leaves
+// deviations either way.
+template <int D, int ST, int R, bool DEV, typename T, typename COEF>
+__device__ __forceinline__ void known_wall(T* f, T win, T den, const COEF& coef) {
+#pragma clang fp contract(off)
+    constexpr int Q = lq(D);
+    if constexpr (DEV) {
+        T rin = win;
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (wall_class(D, R, q) == 1) rin += f[q];
+        const T rw = rin * den;
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            if (wall_class(D, R, q) == 3) f[q] = fma_t(rw, coef(q), -T(wgt(D, q)));
+            if (wall_class(D, R, q) == 2) f[q] = fma_t(rw, coef(q), f[opp(D, q)]);
+        }
+    } else {
+        T rin = T(0);
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (wall_class(D, R, q) == 1) {
+                if constexpr (ST != MPLBHIP_STORE_F64) f[q] += T(wgt(D, q));
+                rin += f[q];
+            }
+        const T rw = T(2) * rin / den;
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const T wr = T(wgt(D, q)) * rw;
+            if (wall_class(D, R, q) == 3) f[q] = wr * coef(q);
+            if (wall_class(D, R, q) == 2) f[q] = wr * coef(q) + f[opp(D, q)];
+        }
+        if constexpr (ST != MPLBHIP_STORE_F64) {
+#pragma unroll
+            for (int q = 0; q < Q; q++) f[q] -= T(wgt(D, q));
+        }
+    }
+}
+
+// The bits of wall_class 1 of a region; class 2 are the opposite ones, as
+// every wall region has them.
+template <int D> __host__ __device__ constexpr uint32_t wall_in(int r) {
+    uint32_t m = 0;
+    for (int q = 0; q < lq(D); q++)
+        if (wall_class(D, r, q) == 1) m |= 1u << q;
+    return m;
+}
+
+// known_wall for lanes of different regions at once, by the lane's wall_in
+// mask (0: no wall, f stays) and values: the lanes of a corner tile take one
+// pass and one division instead of one each per face and corner.
+template <int D, int ST, typename T>
+__device__ __forceinline__ void lane_wall(T* f, uint32_t in, T win, T den, const T* c) {
+#pragma clang fp contract(off)
+    constexpr int Q = lq(D);
+    T rin = ST == MPLBHIP_STORE_F64 ? T(0) : win;
+#pragma unroll
+    for (int q = 1; q < Q; q++) rin += (in >> q & 1u) ? f[q] : T(0);
+    const T rw = ST == MPLBHIP_STORE_F64 ? T(2) * rin / den : rin * den;
+    const bool wall = in != 0;
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int p = opp(D, q);
+        if (p < q) continue;
+        const bool qi = in >> q & 1u, pi = in >> p & 1u;
+        if constexpr (ST == MPLBHIP_STORE_F64) {
+            const T wr = T(wgt(D, q)) * rw;
+            const T vq = wr * c[q] + (pi ? f[p] : T(0)), vp = wr * c[p] + (qi ? f[q] : T(0));
+            f[q] = wall && !qi ? vq : f[q];
+            if (p != q) f[p] = wall && !pi ? vp : f[p];
+        } else {
+            const T w = -T(wgt(D, q));
+            const T vq = fma_t(rw, c[q], pi ? f[p] : w), vp = fma_t(rw, c[p], qi ? f[q] : w);
+            f[q] = wall && !qi ? vq : f[q];
+            if (p != q) f[p] = wall && !pi ? vp : f[p];
+        }
+    }
+}
+
 // rescale part of KerCutCellExtrapolPressure1ST[3D]
 // (boundary_kernel.inc:404-488, 894-1182); f already holds the copied
 // populations.  The loop stops before the last population (:484, :1178).
@@ -516,9 +610,9 @@ struct NodeStore {
 // collision, whose new populations go to `store` (population, value in
 // storage units).  f holds full values when `full` (boundary path), else
 // (reduced storage) deviations g = f - w.
-// GENERAL: whether the case may have a body force or run
-// Collision_BGKThermal4th (FP64).
-template <int D, int ST, int MODE, bool GENERAL = true, typename SINK = NodeStore<ST, false>>
+// EXTRA: what the case may have besides plain BGK: 0 nothing, 1 a body force,
+// 2 that and Collision_BGKThermal4th (FP64).
+template <int D, int ST, int MODE, int EXTRA = 2, typename SINK = NodeStore<ST, false>>
 __device__ __forceinline__ void finish_node(const KParams& kp, const BlockParams& B,
                                             typename Store<ST>::T* f, bool full,
                                             bool force_node, int64_t mnode, const SINK& store,
@@ -545,7 +639,7 @@ __device__ __forceinline__ void finish_node(const KParams& kp, const BlockParams
                 if (cvel(D, q, d) < 0) u -= kCS * f[q];
             }
             u /= rho;
-            if (GENERAL && kp.force_macros && force_node) u += (B.dt * B.g[d] / 2);
+            if (EXTRA > 0 && kp.force_macros && force_node) u += (B.dt * B.g[d] / 2);
             uvw[d] = u;
         }
         if constexpr (MODE == MODE_MATERIALIZE || MODE == MODE_STEP_CHECK) {
@@ -572,7 +666,7 @@ __device__ __forceinline__ void finish_node(const KParams& kp, const BlockParams
 #pragma unroll
                 for (int q = 0; q < Q; q++) kp.fhost[h + q * nn] = f[q];
             }
-        } else if (GENERAL && kp.thermal) {
+        } else if (EXTRA == 2 && kp.thermal) {
             // KerCollideBGKThermal[3D] (model_kernel.inc:267-310, 457-502):
             // tau = tauRef / (rho sqrt(T)) per node, the 4th-order
             // equilibrium at T, and f - w (f - feq) (+ tau w F)
@@ -597,7 +691,7 @@ __device__ __forceinline__ void finish_node(const KParams& kp, const BlockParams
         } else {
             // BGK collision with the optional first-order force source
             const double tw = B.tau_omega, om1 = B.one_minus_omega;
-            const bool addf = GENERAL && force_node && kp.force_type == 1;
+            const bool addf = EXTRA > 0 && force_node && kp.force_type == 1;
             // CalcBGKFeq (feq_ref) with the same operations on the same
             // values in the same order: terms with c = 0 add a zero and are
             // left out, and an opposite velocity's cu is the exact negative,
@@ -663,7 +757,7 @@ __device__ __forceinline__ void finish_node(const KParams& kp, const BlockParams
 #pragma unroll
         for (int d = 0; d < ldim(D); d++) {
             ul[d] = j[d] * inv;
-            if (GENERAL && kp.force_macros && force_node) ul[d] = __builtin_fmaf(j[d], inv, B.fhalf_dtg[d]);
+            if (EXTRA > 0 && kp.force_macros && force_node) ul[d] = __builtin_fmaf(j[d], inv, B.fhalf_dtg[d]);
         }
         float usq = __builtin_fmaf(ul[0], ul[0], ul[1] * ul[1]);
         if constexpr (ldim(D) == 3) usq = __builtin_fmaf(ul[2], ul[2], usq);
@@ -695,7 +789,7 @@ __device__ __forceinline__ void finish_node(const KParams& kp, const BlockParams
             }
         } else {
             const float om = B.fomega, om1 = B.fone_minus_omega;
-            const bool addf = GENERAL && force_node && kp.force_type == 1;
+            const bool addf = EXTRA > 0 && force_node && kp.force_type == 1;
             const float c0 = __builtin_fmaf(rho, -1.5f * usq, drho);
             if constexpr (ST == MPLBHIP_STORE_F16) {
                 // g' = (1 - om) g + om geq in storage units h = g / s_q

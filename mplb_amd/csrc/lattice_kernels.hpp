@@ -133,6 +133,25 @@ struct PairBlock {
     int32_t div_sh[2];
 };
 
+// Several steps in one launch of 2D blocks (k_march): one wave's share.  Its
+// lanes form groups of `group` lanes, each over `group` * C columns from x0
+// on; group g marches through the rows of chunk chunk0 + g (rows of them).
+struct MarchWave {
+    int32_t block;
+    int32_t x0;      // first column
+    int32_t xs, xe;  // columns it stores
+    int32_t group;
+    int32_t chunk0, rows;
+    int32_t first;   // 1: the wave that records the block's parity
+};
+
+// Several steps in one launch of small 2D blocks (k_tile): one workgroup's
+// tile, its first node.
+struct TileWG {
+    int32_t block, x0, y0;
+    int32_t first;   // 1: the workgroup that records the block's parity
+};
+
 struct KParams {
     const BlockParams* blocks;
     int32_t nblocks;
@@ -191,6 +210,13 @@ struct KParams {
     const int32_t* wg_block_pair;
     int32_t npair;
     int32_t pair_nt;
+    const MarchWave* march;
+    int32_t nmarch;
+    const TileWG* tile;
+    int32_t ntile2d;
+    int32_t tile_row;    // tiles per row (one block)
+    int32_t tile_steps;  // steps of this launch
+    int32_t wrap_x;      // the blocks are linked to themselves along x
 };
 
 struct HaloParams {

@@ -25,6 +25,11 @@ hipError_t launch_lattice(int dim, int storage, int mode, const KParams& kp,
 hipError_t launch_materialize_split(int dim, int storage, const KParams& kp, hipStream_t s);
 bool pair_shape(int storage, int nt, int* positions);
 hipError_t launch_pair(int lat, int storage, const KParams& kp, hipStream_t s);
+bool march_shape(int storage, bool obst, int* steps);
+hipError_t launch_march(int storage, const KParams& kp, hipStream_t s);
+int tile_max_steps(int side);
+void tile_wall_classes(int region, uint32_t* in, uint32_t* out, uint32_t* par);
+hipError_t launch_tile(int storage, int side, const KParams& kp, hipStream_t s);
 hipError_t launch_halo(const HaloParams& hp, hipStream_t s);
 hipError_t launch_halo_multi(const HaloParams* links, const int32_t* wg_start, int nlinks,
                              int nwg, int Q, int elem_bytes, hipStream_t s);
@@ -135,6 +140,19 @@ struct mplbhip_ctx {
     std::vector<int32_t> wg_pair_host;
     int npair = 0, pair_nt = 0;
     DevBuf dpair, wg_pair;
+    // several steps per launch of 2D blocks (k_march), likewise: steps of the
+    // form, every wave's share
+    bool march_ok = false, march = false;
+    int march_steps = 0;
+    std::vector<MarchWave> march_host;
+    DevBuf dmarch;
+    // several steps per launch of small 2D blocks (k_tile): the tiles, their
+    // side, and whether the blocks are linked to themselves along x
+    bool tile_ok = false, tile = false, wrap_x = false;
+    int tile_side = 0, ntile2d = 0, tile_row = 0;
+    std::vector<TileWG> tile_host;
+    DevBuf dtile;
+    bool halo_stale = false;  // the latest fStage's halos are not exchanged
     int singles = 0;  // single steps taken before their launch was tuned
     std::vector<BndSeg> segs;
     std::vector<std::vector<uint8_t>> solid;  // obstacle nodes per block (empty: none)
@@ -323,6 +341,12 @@ static KParams base_params(mplbhip_ctx* c) {
     kp.wg_block_pair = static_cast<const int32_t*>(c->wg_pair.p);
     kp.npair = c->npair;
     kp.pair_nt = c->pair_nt;
+    kp.march = static_cast<const MarchWave*>(c->dmarch.p);
+    kp.nmarch = (int)c->march_host.size();
+    kp.tile = static_cast<const TileWG*>(c->dtile.p);
+    kp.ntile2d = c->ntile2d;
+    kp.tile_row = c->tile_row;
+    kp.wrap_x = c->wrap_x ? 1 : 0;
     return kp;
 }
 
@@ -417,10 +441,20 @@ static int enqueue_swap_step(mplbhip_ctx* c, bool check, bool residual) {
 // or one whole-lattice launch's tiles (small cases, the swap scheme)
 static int reduce_split(const mplbhip_ctx* c) { return c->fused || c->swap ? 0 : 1; }
 
+// the halo copies that a launch of several steps left out (k_tile wraps by
+// itself), ahead of a kernel that reads them
+static int fresh_halos(mplbhip_ctx* c) {
+    if (c->halo_stale)
+        if (int rc = exchange(c, c->cur)) return rc;
+    c->halo_stale = false;
+    return 0;
+}
+
 // one step from parity c->cur (step kernels, then the halo copies, which
 // wait for both kernels); leaves c->cur flipped
 static int enqueue_step(mplbhip_ctx* c, bool check, bool residual) {
     if (c->swap) return enqueue_swap_step(c, check, residual);
+    if (int rc = fresh_halos(c)) return rc;
     KParams kp = base_params(c);
     kp.want_residual = residual ? 1 : 0;
     const int mode = check ? MODE_STEP_CHECK : MODE_STEP;
@@ -430,18 +464,28 @@ static int enqueue_step(mplbhip_ctx* c, bool check, bool residual) {
     return 0;
 }
 
-// two steps in one launch from parity c->cur; leaves c->cur flipped.  The
-// other fStage buffer then holds the state two steps back, so a run whose
-// result is measured by re-streaming ends with a single step.
-static int enqueue_pair(mplbhip_ctx* c) {
-    HIPCHK(c, launch_pair(c->lat, c->storage, base_params(c), c->stream));
-    c->cur ^= 1;
-    return 0;
+// steps per launch in force (1: single steps); a body force given after
+// prepare turns the forms without one off
+static int launch_steps(const mplbhip_ctx* c) {
+    if (c->swap || c->thermal) return 1;
+    if (c->tile) return tile_max_steps(c->tile_side);
+    if (c->force_type || c->force_macros) return 1;
+    return c->pair ? 2 : c->march ? c->march_steps : 1;
 }
 
-// two-step launches in force: a body force given after prepare turns them off
-static bool use_pair(const mplbhip_ctx* c) {
-    return c->pair && !c->force_type && !c->force_macros;
+// n steps in one launch from parity c->cur (launch_steps(c); k_tile also
+// takes fewer); leaves c->cur flipped.  The other fStage buffer then holds
+// the state n steps back, so a run whose result is measured by re-streaming
+// ends with a single step.
+static int enqueue_multi(mplbhip_ctx* c, int n) {
+    KParams kp = base_params(c);
+    kp.tile_steps = n;
+    if (c->tile) HIPCHK(c, launch_tile(c->storage, c->tile_side, kp, c->stream));
+    else if (c->pair) HIPCHK(c, launch_pair(c->lat, c->storage, kp, c->stream));
+    else HIPCHK(c, launch_march(c->storage, kp, c->stream));
+    c->halo_stale = !c->halos.empty();
+    c->cur ^= 1;
+    return 0;
 }
 
 static int build_graphs(mplbhip_ctx* c, int nsteps) {
@@ -451,10 +495,9 @@ static int build_graphs(mplbhip_ctx* c, int nsteps) {
         const int saved = c->cur;
         c->cur = p;
         int rc = 0;
-        if (use_pair(c))
-            for (int s = 0; s < nsteps && rc == 0; s += 2) rc = enqueue_pair(c);
-        else
-            for (int s = 0; s < nsteps && rc == 0; s++) rc = enqueue_step(c, false, false);
+        const int ls = launch_steps(c);
+        for (int s = 0; s < nsteps && rc == 0; s += ls)
+            rc = ls > 1 ? enqueue_multi(c, ls) : enqueue_step(c, false, false);
         c->cur = saved;
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(c->stream, &g);
@@ -1407,6 +1450,149 @@ static void pair_tiling(const int* n, int es, long long nblk, int nt, int np, Pa
     }
 }
 
+// Whether a region is a wall as known_wall and lane_wall have it: masked
+// pulls and one EQM application with the classes of its place.
+static bool plain_wall2(const RegionProg& P, int r) {
+    if (P.kind != RK_MASKED || P.nops != 1 || P.op[0].type != OP_EQM || P.persist >= 0)
+        return false;
+    uint32_t in, out, par;
+    tile_wall_classes(r, &in, &out, &par);
+    const BCOp& op = P.op[0];
+    return op.m_in == in && op.m_out == out && op.m_par == par;
+}
+
+// Whether the case can take several steps per launch of k_march: 2D blocks
+// without connections, BGK without a body force, every envelope region a
+// wall.
+static bool march_allowed(const mplbhip_ctx* c) {
+    if (c->dim != 2 || c->swap || c->thermal || !c->plan.links.empty()) return false;
+    // (a block is one buffer resource, of 32-bit byte offsets)
+    for (const BlockParams& B : c->bp)
+        if ((int64_t)B.sz * (int64_t)c->es >= (int64_t)1 << 31) return false;
+    for (size_t b = 0; b < c->plan.blocks.size(); b++)
+        for (int r = 1; r < c->plan.nregions; r++)
+            if (!plain_wall2(c->plan.progs[b * c->plan.nregions + r], r)) return false;
+    return true;
+}
+
+// Whether the case can run in tiles (k_tile): such blocks, with or without a
+// body force, or blocks without obstacles that are linked to themselves along
+// x (their x faces pull every population) and long enough to wrap once.
+static bool tile_allowed(mplbhip_ctx* c) {
+    if (c->dim != 2 || c->swap || c->thermal) return false;
+    std::vector<int> sides(c->plan.blocks.size(), 0);
+    for (const LinkDesc& l : c->plan.links) {
+        if (l.rot || l.from != l.to) return false;
+        if (l.fsurf == BS_Left && l.tsurf == BS_Right) sides[l.from] |= 1;
+        else if (l.fsurf == BS_Right && l.tsurf == BS_Left) sides[l.from] |= 2;
+        else return false;
+    }
+    c->wrap_x = !c->plan.links.empty();
+    if (c->wrap_x && !c->obst.empty()) return false;
+    for (size_t b = 0; b < c->plan.blocks.size(); b++) {
+        if (sides[b] != (c->wrap_x ? 3 : 0)) return false;
+        if (c->wrap_x && c->bp[b].n[0] < 32) return false;
+        for (int r = 1; r < c->plan.nregions; r++) {
+            const RegionProg& P = c->plan.progs[b * c->plan.nregions + r];
+            if (c->wrap_x && r < 3) {
+                if (P.kind != RK_FULL || P.nops != 0 || P.persist >= 0) return false;
+            } else if (!plain_wall2(P, r)) {
+                return false;
+            }
+        }
+    }
+    return true;
+}
+
+static int upload_table(mplbhip_ctx* c, DevBuf& d, const void* v, size_t bytes) {
+    if (d.bytes < bytes)
+        if (int rc = dalloc(c, d, bytes)) return rc;
+    HIPCHK(c, hipMemcpyAsync(d.p, v, bytes, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+}
+
+// the tiles of k_tile; a single block's follow from the workgroup's number
+static int assign_tiles2d(mplbhip_ctx* c, bool only_active) {
+    auto count = [&](int w) {
+        c->tile_side = w;
+        c->tile_row = (c->bp[0].n[0] + w - 1) / w;
+        c->ntile2d = 0;
+        for (const BlockParams& B : c->bp)
+            if (!only_active || B.active)
+                c->ntile2d += ((B.n[0] + w - 1) / w) * ((B.n[1] + w - 1) / w);
+        return c->ntile2d;
+    };
+    if (count(8) > 256 && count(16) > 768) count(24);
+    if (c->bp.size() == 1) return 0;
+    const int w = c->tile_side;
+    c->tile_host.clear();
+    for (size_t b = 0; b < c->bp.size(); b++) {
+        const BlockParams& B = c->bp[b];
+        if (only_active && !B.active) continue;
+        for (int y = 0; y < B.n[1]; y += w)
+            for (int x = 0; x < B.n[0]; x += w)
+                c->tile_host.push_back(TileWG{(int32_t)b, x, y, x == 0 && y == 0});
+    }
+    return upload_table(c, c->dtile, c->tile_host.data(), c->tile_host.size() * sizeof(TileWG));
+}
+
+// The waves of k_march.  Rows per chunk: 16 read and compute 2K of K + 16
+// rows again, 8 twice that share, for twice the waves.
+// (us per step with 8, 12, 16 rows: FP32 1024^2 10.1, 10.4, 11.2; 1448^2 16.5,
+// 16.3, 15.9; 2048^2 27.7, 26.4, 25.0; FP64 1024^2 18.1, 17.7, 18.7)
+static int assign_march(mplbhip_ctx* c, bool only_active) {
+    march_shape(c->storage, !c->obst.empty(), &c->march_steps);
+    const int K = c->march_steps, own = 64 - 2 * K;
+    auto group = [&](int nx) { return nx <= 16 ? 16 : nx <= 32 ? 32 : 64; };
+    // strips: the first and the last one need no margin on the wall's side
+    auto strips = [&](int nx) { return nx <= 64 ? 1 : (nx - 64 + own - 1) / own + 1; };
+    auto list = [&](int rows) {
+        c->march_host.clear();
+        for (size_t b = 0; b < c->bp.size(); b++) {
+            const BlockParams& B = c->bp[b];
+            if (only_active && !B.active) continue;
+            const int G = group(B.n[0]), T = strips(B.n[0]), chunks = (B.n[1] + rows - 1) / rows;
+            for (int t = 0; t < T; t++)
+                for (int k = 0; k < chunks; k += 64 / G) {
+                    MarchWave M;
+                    M.block = (int32_t)b;
+                    M.x0 = t * own;
+                    M.xs = t ? M.x0 + K : 0;
+                    M.xe = t + 1 < T ? M.x0 + 64 - K : B.n[0];
+                    M.group = G;
+                    M.chunk0 = k;
+                    M.rows = rows;
+                    M.first = t == 0 && k == 0;
+                    c->march_host.push_back(M);
+                }
+        }
+        return (int)c->march_host.size();
+    };
+    if (list(16) < 2048) list(8);
+    return upload_table(c, c->dmarch, c->march_host.data(), c->march_host.size() * sizeof(MarchWave));
+}
+
+// The several-step form of 2D cases over the (active) blocks, by measured
+// steps (us, cavities of n^2 nodes; single steps, tiles, march):
+//   FP64  512: 16.1, 6.3, 8.6   1024: 26.2, 16.0, 17.7   1448: -, 29.0, 28.7
+//   FP32  512: 14.0, 3.9, 6.0    860: -, 8.3, 8.5        1024: 17.3, 10.6, 10.1
+// so tiles up to 2^20 nodes in FP64 and below that in reduced storage, where
+// k_march reads less per node, and above it where k_march cannot run
+// (2048 x 1024 periodic channel, single against tiles: FP64 57.4 and 43.2,
+// FP32 34.0 and 18.9).  The tile's side by the number of workgroups: small
+// ones while the chip has a CU for each (128^2 FP64: 1.7 with side 8, 2.2
+// with 16; 192^2: 3.1 and 2.5), the large, four-step ones when there are
+// several rounds of them (400^2 FP32: 3.1 either way; 512^2 FP64: 6.7 with
+// 16, 6.3 with 24).
+static int assign_2d(mplbhip_ctx* c, bool only_active) {
+    const int64_t most = c->storage == MPLBHIP_STORE_F64 ? 1 << 20 : (1 << 20) - 1;
+    c->tile = c->tile_ok && c->pair_env >= 0 && c->pair_env != 2 &&
+              (c->grid_nodes <= most || !c->march_ok);
+    c->march = c->march_ok && c->pair_env >= 0 && !c->tile;
+    return c->tile ? assign_tiles2d(c, only_active) : c->march ? assign_march(c, only_active) : 0;
+}
+
 // Two-step launches over the (active) blocks: from 2^16 nodes on.  Below, a
 // step is bound by the launch and its latency either way (32^3 FP64: 11.1 us
 // per step against 9.8 in one whole-lattice launch; 48^3: 14.0 against 21.8).
@@ -1675,8 +1861,11 @@ int mplbhip_prepare(mplbhip_ctx* c) {
     // a single-step form chosen by the environment is the one that runs
     c->pair_ok = pair_allowed(c);
     c->pair_env = c->fused_env || c->fold_env || c->xgroup_env || c->h2_env || c->xcd_remap ? -1 : 0;
-    if (const char* e = std::getenv("MPLBHIP_PAIR")) c->pair_env = std::atoi(e) != 0 ? 1 : -1;
+    if (const char* e = std::getenv("MPLBHIP_PAIR")) c->pair_env = std::atoi(e) > 0 ? std::atoi(e) : -1;
     if (int rc = assign_pairs(c, false)) return rc;
+    c->march_ok = march_allowed(c);
+    c->tile_ok = tile_allowed(c);
+    if (int rc = assign_2d(c, false)) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -1918,6 +2107,7 @@ static int first_collision(mplbhip_ctx* c) {
     for (int i = 0; i < 2; i++)
         HIPCHK(c, launch_fill(c->parity[i].p, (int64_t)c->parity[i].bytes, c->stream));
     c->cur = 0;
+    c->halo_stale = false;
     KParams kp = base_params(c);
     int mode = MODE_INIT_FEQ;
     if (c->init_from_f) {
@@ -1938,12 +2128,14 @@ static int first_collision(mplbhip_ctx* c) {
     }
     HIPCHK(c, launch_lattice(c->lat, c->storage, mode, kp, c->stream));
     if (int rc = exchange(c, 0)) return rc;
-    // with two-step launches the single ones only end a run: not tuned yet
-    return use_pair(c) ? 0 : autotune(c);
+    // beside launches of several steps the single ones only end a run: not
+    // tuned yet
+    return launch_steps(c) > 1 ? 0 : autotune(c);
 }
 
+// tail: a check step follows, so the last step need not be a single one
 static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
-                     double* ms_kernel) {
+                     double* ms_kernel, bool tail = false) {
     if (int rc = need_device(c)) return rc;
     if (int rc = ensure_init(c)) return rc;
     if (nsteps < 0) return fail(c, MPLBHIP_ERR_ARG, "negative step count");
@@ -1953,6 +2145,7 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
     double ktot = 0.0;
     if (timed) {
         if (int rc = autotune(c)) return rc;
+        if (int rc = fresh_halos(c)) return rc;
         // per-step events bracket the bulk kernel and the boundary kernel,
         // each on the stream it runs on (the step's own launch structure)
         std::vector<hipEvent_t> evs(4 * (size_t)nsteps);
@@ -2013,28 +2206,30 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         if (g >= 2 && g <= 1024 && g % 2 == 0) G = g;
     }
     int left = nsteps;
-    // two-step launches leave the last step to a single one
-    const bool pair = use_pair(c);
-    const int keep = pair ? 1 : 0;
-    if (left - keep >= G) {
+    // launches of several steps leave the last step to a single one
+    const int ls = launch_steps(c), keep = ls > 1 && !tail ? 1 : 0;
+    G -= G % ls;  // whole launches
+    if (G > 0 && left - keep >= G) {
         if (c->graph_steps != G)
             if (int rc = build_graphs(c, G)) return rc;
         while (left - keep >= G) {
             HIPCHK(c, hipGraphLaunch(c->gexec[c->cur], c->stream));
-            // G is even: single steps leave the parity unchanged
-            if (pair && (G / 2) % 2) c->cur ^= 1;
+            // every launch flips the parity
+            if ((G / ls) % 2) c->cur ^= 1;
+            c->halo_stale = ls > 1 && !c->halos.empty();
             c->tstep += G;
             left -= G;
         }
     }
-    while (pair && left - keep >= 2) {
-        if (int rc = enqueue_pair(c)) return rc;
-        c->tstep += 2;
-        left -= 2;
+    while (ls > 1 && left - keep >= (c->tile ? 2 : ls)) {
+        const int n = std::min(ls, left - keep);
+        if (int rc = enqueue_multi(c, n)) return rc;
+        c->tstep += n;
+        left -= n;
     }
     while (left > 0) {
         // a program that takes its steps one at a time gets them tuned too
-        if (pair && !c->tuned && ++c->singles > 64)
+        if (ls > 1 && !c->tuned && ++c->singles > 64)
             if (int rc = autotune(c)) return rc;
         if (int rc = enqueue_step(c, false, false)) return rc;
         c->tstep++;
@@ -2060,7 +2255,9 @@ int mplbhip_iterate(mplbhip_ctx* c, double criteria, int check_period,
         long long plain = std::min<long long>(to_check, max_steps - done);
         while (plain > 0) {
             const int chunk = (int)std::min<long long>(plain, 1 << 20);
-            if (int rc = run_steps(c, chunk, false, nullptr, nullptr)) return rc;
+            if (int rc = run_steps(c, chunk, false, nullptr, nullptr,
+                                   plain == chunk && done + chunk < max_steps))
+                return rc;
             plain -= chunk;
             done += chunk;
         }
@@ -2129,7 +2326,8 @@ static int compact_grid(mplbhip_ctx* c, bool on) {
     c->fused = c->fused_env ? c->fused_full
                             : (on ? c->grid_nodes < (1 << 18) : c->fused_full);
     drop_graphs(c);
-    return assign_pairs(c, on);
+    if (int rc = assign_pairs(c, on)) return rc;
+    return assign_2d(c, on);
 }
 
 // Restart the listed blocks at rest, as a rest start forms its first
@@ -2211,7 +2409,9 @@ int mplbhip_iterate_batch(mplbhip_ctx* c, double criteria, int check_period,
         long long plain = std::min<long long>(to_check, max_steps - done);
         while (plain > 0) {
             const int chunk = (int)std::min<long long>(plain, 1 << 20);
-            if (int rc = run_steps(c, chunk, false, nullptr, nullptr)) return rc;
+            if (int rc = run_steps(c, chunk, false, nullptr, nullptr,
+                                   plain == chunk && done + chunk < max_steps))
+                return rc;
             plain -= chunk;
             done += chunk;
         }

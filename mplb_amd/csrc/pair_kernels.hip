@@ -85,62 +85,16 @@ __device__ __forceinline__ double bit_or(double a, double b) {
                               __builtin_bit_cast(int64_t, a) | __builtin_bit_cast(int64_t, b));
 }
 
-// FindBdyDvType3D (boundary_host_device.h:191-706) of a face or an edge
-// region: 1 streams into the wall, 2 comes out of it, 3 along it
-__host__ __device__ constexpr int wall_class(int D, int r, int q) {
-    const int code[3] = {r % 3, r / 3 % 3, r / 9};
-    int n = 0, cn[3] = {0, 0, 0};
-    for (int a = 0; a < 3; a++)
-        if (code[a]) cn[n++] = (code[a] == 1 ? 1 : -1) * cvel(D, q, a);
-    if (n == 1) return cn[0] < 0 ? 1 : cn[0] > 0 ? 2 : 3;
-    if ((cn[0] <= 0 && cn[1] < 0) || (cn[0] < 0 && cn[1] == 0)) return 1;
-    if ((cn[0] >= 0 && cn[1] > 0) || (cn[0] > 0 && cn[1] == 0)) return 2;
-    return 3;
-}
-
 // pair_boundary of a face or edge whose populations' classes are known at
-// compile time: the faces, and the edges that every plane has.  (Every
-// incoming population is a pulled one, and every other is written.)  The
-// general form issues about 350 instructions; one wave per tile runs it
-// while the others wait at the barrier, 0.09 of 0.27 ms per step for the
-// four z edges of D3Q19 FP32 256^3 alone.
+// compile time: the faces, and the edges that every plane has.  The general
+// form issues about 350 instructions; one wave per tile runs it while the
+// others wait at the barrier, 0.09 of 0.27 ms per step for the four z edges
+// of D3Q19 FP32 256^3 alone.
 template <int D, int ST, int R>
 __device__ __forceinline__ void pair_wall(PairWalls<D, typename Store<ST>::T>& W,
                                           typename Store<ST>::T* f) {
-#pragma clang fp contract(off)
-    using T = typename Store<ST>::T;
-    constexpr int Q = lq(D);
-    if constexpr (ST == MPLBHIP_STORE_F16) {
-        T rin = W.win[R];
-#pragma unroll
-        for (int q = 0; q < Q; q++)
-            if (wall_class(D, R, q) == 1) rin += f[q];
-        const T rw = rin * W.den[R];
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-            if (wall_class(D, R, q) == 3) f[q] = fma_t(rw, W.c[R][q], -T(wgt(D, q)));
-            if (wall_class(D, R, q) == 2) f[q] = fma_t(rw, W.c[R][q], f[opp(D, q)]);
-        }
-        return;
-    }
-    T rin = T(0);
-#pragma unroll
-    for (int q = 0; q < Q; q++)
-        if (wall_class(D, R, q) == 1) {
-            if constexpr (ST != MPLBHIP_STORE_F64) f[q] += T(wgt(D, q));
-            rin += f[q];
-        }
-    const T rw = T(2) * rin / W.den[R];
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-        const T wr = T(wgt(D, q)) * rw;
-        if (wall_class(D, R, q) == 3) f[q] = wr * W.c[R][q];
-        if (wall_class(D, R, q) == 2) f[q] = wr * W.c[R][q] + f[opp(D, q)];
-    }
-    if constexpr (ST != MPLBHIP_STORE_F64) {
-#pragma unroll
-        for (int q = 0; q < Q; q++) f[q] -= T(wgt(D, q));
-    }
+    known_wall<D, ST, R, ST == MPLBHIP_STORE_F16>(
+        f, W.win[R], W.den[R], [&](int q) { return W.c[R][q]; });
 }
 
 // The boundary program of region r (not the interior) on a lane's gathered
@@ -406,7 +360,7 @@ __global__ __launch_bounds__(NT, ST == MPLBHIP_STORE_F64 ? 2 : 4) void k_pair(KP
             const int r = rc1 + 9 * region_code(k, nz);
             if (r && n1.valid)
                 pair_boundary<D, ST, false>(s_w, r, f, own1 && k >= zs && k < ze, per_next);
-            finish_node<D, ST, MODE_STEP, false>(kp, B, f, false, true, 0, RegSink<ST>{h}, n1.x,
+            finish_node<D, ST, MODE_STEP, 0>(kp, B, f, false, true, 0, RegSink<ST>{h}, n1.x,
                                                  n1.y, k, acc);
         }
         // the second step of the plane before has read what is replaced
@@ -445,7 +399,7 @@ __global__ __launch_bounds__(NT, ST == MPLBHIP_STORE_F64 ? 2 : 4) void k_pair(KP
             const int r = rc2 + 9 * region_code(z, nz);
             if (r && on) pair_boundary<D, ST, true>(s_w, r, f, true, per_next);
             E o[Q];
-            finish_node<D, ST, MODE_STEP, false>(kp, B, f, false, true, 0, RegSink<ST>{o}, n2.x,
+            finish_node<D, ST, MODE_STEP, 0>(kp, B, f, false, true, 0, RegSink<ST>{o}, n2.x,
                                                  n2.y, z, acc);
             // nontemporal rows, except in tiles whose x-face nodes another
             // wave stores: those lines meet in L2
