@@ -217,6 +217,10 @@ struct KParams {
     int32_t tile_row;    // tiles per row (one block)
     int32_t tile_steps;  // steps of this launch
     int32_t wrap_x;      // the blocks are linked to themselves along x
+    // the swap scheme: the buffer written (0 but within a run of k_swap_pull),
+    // and the masks of every block's regions
+    int32_t swap_to;
+    const uint2* swap_mask;
 };
 
 struct HaloParams {

@@ -41,6 +41,8 @@ hipError_t launch_lift(int dim, const KParams& kp, int64_t nodes, hipStream_t s)
 hipError_t launch_rest_macros(const KParams& kp, int b, int64_t nodes, hipStream_t s);
 hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t s);
 hipError_t scratch_address(double** ptr);
+bool swap_masks(const RegionProg* progs, uint32_t* mask);
+hipError_t launch_swap_pull(const KParams& kp, int nbnd, bool collide, bool large, hipStream_t s);
 hipError_t launch_swap(int part, const KParams& kp, int nbnd, hipStream_t s);
 }  // namespace mplbhip
 
@@ -86,6 +88,10 @@ struct mplbhip_ctx {
     // swap_formed once f^0 is in it
     bool swap = false;
     bool swap_formed = false;
+    // the case runs k_swap_pull, whose steps between a run's first collision
+    // and its last stream leave the collided lattice in fs[cur]
+    bool swap_pull = false, swap_run = false;
+    DevBuf swap_mask;
     bool init_from_f = false;
     bool init_lift = false;  // f^0 = feq + first-order non-equilibrium part
     long long tstep = 0;
@@ -347,6 +353,7 @@ static KParams base_params(mplbhip_ctx* c) {
     kp.ntile2d = c->ntile2d;
     kp.tile_row = c->tile_row;
     kp.wrap_x = c->wrap_x ? 1 : 0;
+    kp.swap_mask = static_cast<const uint2*>(c->swap_mask.p);
     return kp;
 }
 
@@ -420,11 +427,43 @@ static int launch_step_kernels(mplbhip_ctx* c, const KParams& kp, int mode,
     return 0;
 }
 
+// A run of the swap scheme's one-pass forms: the collision of f (fs[0]) into
+// the buffer from which the run's passes end in fs[0] again, a pass of
+// k_swap_pull per step, the last of which streams and applies the walls only.
+static int swap_begin(mplbhip_ctx* c, int passes) {
+    KParams kp = base_params(c);
+    kp.swap_to = c->cur = passes & 1;
+    HIPCHK(c, launch_swap(0, kp, 0, c->stream));
+    c->swap_run = true;
+    return 0;
+}
+static int swap_pass(mplbhip_ctx* c, bool collide) {
+    KParams kp = base_params(c);
+    kp.swap_to = 1 - c->cur;
+    HIPCHK(c, launch_swap_pull(kp, c->nbnd_v[0], collide, c->fs[0].bytes > ((size_t)1 << 28),
+                               c->stream));
+    c->cur ^= 1;
+    return 0;
+}
+static int swap_end(mplbhip_ctx* c) {
+    c->swap_run = false;
+    return swap_pass(c, false);
+}
+
 // SwapStreamCollision (evolution.cpp:195-252) on the one lattice f:
 // collision and force, halo exchange of f, local swap, swap stream,
 // boundaries; with check, the macros (and residual partials) of the result
 static int enqueue_swap_step(mplbhip_ctx* c, bool check, bool residual) {
     KParams kp = base_params(c);
+    if (c->swap_pull) {
+        if (int rc = swap_begin(c, 1)) return rc;
+        if (int rc = swap_end(c)) return rc;
+        if (check) {
+            kp.want_residual = residual ? 1 : 0;
+            HIPCHK(c, launch_swap(5, kp, 0, c->stream));
+        }
+        return 0;
+    }
     HIPCHK(c, launch_swap(0, kp, 0, c->stream));
     if (int rc = exchange(c, 0)) return rc;
     HIPCHK(c, launch_swap(1, kp, 0, c->stream));
@@ -453,6 +492,7 @@ static int fresh_halos(mplbhip_ctx* c) {
 // one step from parity c->cur (step kernels, then the halo copies, which
 // wait for both kernels); leaves c->cur flipped
 static int enqueue_step(mplbhip_ctx* c, bool check, bool residual) {
+    if (c->swap_run) return swap_pass(c, true);
     if (c->swap) return enqueue_swap_step(c, check, residual);
     if (int rc = fresh_halos(c)) return rc;
     KParams kp = base_params(c);
@@ -676,8 +716,9 @@ void mplbhip_destroy(mplbhip_ctx* c) {
         dfree(c->blocks);
         dfree(c->partials);
         dfree(c->dsegs);
-        dfree(c->wg_block);
-        dfree(c->dobst);
+        for (DevBuf* d : {&c->wg_block, &c->dpair, &c->wg_pair, &c->dmarch, &c->dtile, &c->swap_mask,
+                          &c->temp, &c->dobst})
+            dfree(*d);
         dfree(c->red);
         dfree(c->fhost);
         dfree(c->parity[0]);
@@ -1593,6 +1634,17 @@ static int assign_2d(mplbhip_ctx* c, bool only_active) {
     return c->tile ? assign_tiles2d(c, only_active) : c->march ? assign_march(c, only_active) : 0;
 }
 
+// the swap scheme in one pass per step (k_swap_pull) where no block is
+// connected and every region allows it
+static int assign_swap(mplbhip_ctx* c) {
+    c->swap_pull = c->swap && c->plan.links.empty();
+    const size_t nb = c->plan.blocks.size();
+    std::vector<uint32_t> mask(c->swap_pull ? nb * 54 : 0);
+    for (size_t b = 0; b < nb && c->swap_pull; b++)
+        c->swap_pull = swap_masks(&c->plan.progs[b * c->plan.nregions], &mask[b * 54]);
+    return c->swap_pull ? upload_table(c, c->swap_mask, mask.data(), mask.size() * 4) : 0;
+}
+
 // Two-step launches over the (active) blocks: from 2^16 nodes on.  Below, a
 // step is bound by the launch and its latency either way (32^3 FP64: 11.1 us
 // per step against 9.8 in one whole-lattice launch; 48^3: 14.0 against 21.8).
@@ -1859,6 +1911,7 @@ int mplbhip_prepare(mplbhip_ctx* c) {
     if (int rc = upload_blocks(c)) return rc;
     if (int rc = upload_merged_halos(c)) return rc;
     // a single-step form chosen by the environment is the one that runs
+    if (int rc = assign_swap(c)) return rc;
     c->pair_ok = pair_allowed(c);
     c->pair_env = c->fused_env || c->fold_env || c->xgroup_env || c->h2_env || c->xcd_remap ? -1 : 0;
     if (const char* e = std::getenv("MPLBHIP_PAIR")) c->pair_env = std::atoi(e) > 0 ? std::atoi(e) : -1;
@@ -2140,6 +2193,7 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
     if (int rc = ensure_init(c)) return rc;
     if (nsteps < 0) return fail(c, MPLBHIP_ERR_ARG, "negative step count");
     HIPCHK(c, hipSetDevice(c->device));
+    c->swap_run = false;
     if (c->tstep == 0)
         if (int rc = first_collision(c)) return rc;
     double ktot = 0.0;
@@ -2206,6 +2260,11 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         if (g >= 2 && g <= 1024 && g % 2 == 0) G = g;
     }
     int left = nsteps;
+    const bool pull = c->swap_pull && left > 0;
+    if (pull) {
+        if (int rc = swap_begin(c, left)) return rc;
+        left--;
+    }
     // launches of several steps leave the last step to a single one
     const int ls = launch_steps(c), keep = ls > 1 && !tail ? 1 : 0;
     G -= G % ls;  // whole launches
@@ -2234,6 +2293,10 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         if (int rc = enqueue_step(c, false, false)) return rc;
         c->tstep++;
         left--;
+    }
+    if (pull) {
+        if (int rc = swap_end(c)) return rc;
+        c->tstep++;
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
