@@ -13,6 +13,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 namespace {
@@ -394,6 +395,25 @@ __global__ __launch_bounds__(64 * kSumWaves) void k_sum_partials(const float* __
     }
 }
 
+// V consecutive floats: 4 where the channel counts are multiples of four and
+// the arrays are aligned for it, else 1
+template <int V> struct Vec;
+template <> struct Vec<1> {
+    float v[1];
+    __device__ static Vec ld(const float* p) { return Vec{{*p}}; }
+    __device__ void st(float* p) const { *p = v[0]; }
+};
+template <> struct Vec<4> {
+    float v[4];
+    __device__ static Vec ld(const float* p) {
+        const float4 f = *reinterpret_cast<const float4*>(p);
+        return Vec{{f.x, f.y, f.z, f.w}};
+    }
+    __device__ void st(float* p) const {
+        *reinterpret_cast<float4*>(p) = float4{v[0], v[1], v[2], v[3]};
+    }
+};
+
 __global__ void k_relu_bwd(const float* __restrict__ dout, const float* __restrict__ out,
                            float* __restrict__ din, int64_t count) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count;
@@ -431,50 +451,82 @@ __global__ void k_pool_bwd(const float* __restrict__ dout, float* __restrict__ d
     }
 }
 
+// Where these two and k_channels had an element per iteration with the 64-bit
+// divisions of its whole index (some 100 instructions each), a workgroup now
+// takes one coarse row or 64 pixels and an item's place in it is one 32-bit
+// division; HBM bounds them.
+
 // nearest 2x upsampling (h, wd: the coarse size) into channels [c0, c0+c)
-// of a tensor with ctot channels, and its adjoint
-__global__ void k_up_fwd(const float* __restrict__ in, float* __restrict__ out, int n, int h,
+// of a tensor with ctot channels, and its adjoint: one coarse row per
+// workgroup and iteration, every coarse value read once.  32 images of 64 x 64
+// x 48 to 128 x 128 x 72: 79.7 -> 20.9 us (6.0 TB/s).
+template <int V>
+__global__ void k_up_fwd(const float* __restrict__ in, float* __restrict__ out, int64_t rows,
                          int wd, int c, int ctot, int c0) {
-    const int H = 2 * h, W = 2 * wd;
-    const int64_t total = (int64_t)n * H * W * c;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int ch = (int)(i % c);
-        const int64_t p = i / c;
-        const int x = (int)(p % W), y = (int)((p / W) % H);
-        const int64_t b = p / ((int64_t)W * H);
-        out[p * ctot + c0 + ch] = in[((b * h + y / 2) * wd + x / 2) * c + ch];
+    const uint32_t cv = (uint32_t)c / V, items = (uint32_t)wd * cv;
+    const int64_t W = 2 * (int64_t)wd;
+    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        // (fine row 2 y of image b is row 2 (b h + y) of all)
+        float* fine = out + 2 * r * W * ctot + c0;
+        const float* coarse = in + r * wd * c;
+        for (uint32_t i = threadIdx.x; i < items; i += blockDim.x) {
+            const uint32_t x = i / cv, k = (i - x * cv) * V;
+            const Vec<V> v = Vec<V>::ld(coarse + (int64_t)i * V);
+            float* f = fine + 2 * (int64_t)x * ctot + k;
+            v.st(f);
+            v.st(f + ctot);
+            v.st(f + W * ctot);
+            v.st(f + W * ctot + ctot);
+        }
     }
 }
 
-__global__ void k_up_bwd(const float* __restrict__ dout, float* __restrict__ din, int n, int h,
+template <int V>
+__global__ void k_up_bwd(const float* __restrict__ dout, float* __restrict__ din, int64_t rows,
                          int wd, int c, int ctot, int c0) {
-    const int W = 2 * wd;
-    const int64_t total = (int64_t)n * h * wd * c;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int ch = (int)(i % c);
-        const int64_t p = i / c;
-        const int x = (int)(p % wd), y = (int)((p / wd) % h);
-        const int64_t b = p / ((int64_t)wd * h);
-        const int64_t f = ((b * 2 * h + 2 * y) * W + 2 * x) * ctot + c0 + ch;
-        const int64_t r = (int64_t)W * ctot;
-        din[i] = (dout[f] + dout[f + ctot]) + (dout[f + r] + dout[f + r + ctot]);
+    const uint32_t cv = (uint32_t)c / V, items = (uint32_t)wd * cv;
+    const int64_t W = 2 * (int64_t)wd;
+    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        const float* fine = dout + 2 * r * W * ctot + c0;
+        float* coarse = din + r * wd * c;
+        for (uint32_t i = threadIdx.x; i < items; i += blockDim.x) {
+            const uint32_t x = i / cv, k = (i - x * cv) * V;
+            const float* f = fine + 2 * (int64_t)x * ctot + k;
+            const Vec<V> a = Vec<V>::ld(f), b = Vec<V>::ld(f + ctot);
+            const Vec<V> d = Vec<V>::ld(f + W * ctot), e = Vec<V>::ld(f + W * ctot + ctot);
+            Vec<V> o;
+#pragma unroll
+            for (int j = 0; j < V; j++) o.v[j] = (a.v[j] + b.v[j]) + (d.v[j] + e.v[j]);
+            o.st(coarse + (int64_t)i * V);
+        }
     }
 }
 
 // copy channels [0, c) of src (c channels) into channels [c0, c0 + c) of
-// dst (ctot channels) (dir = 0), or back (dir = 1), or add them back (dir = 2)
+// dst (ctot channels) (dir = 0), or back (dir = 1), or add them back (dir =
+// 2): 64 pixels per workgroup and iteration.  32 images of 128 x 128 x 24
+// into 72: 19.7 -> 17.3 us (5.8 TB/s).
+template <int V>
 __global__ void k_channels(const float* __restrict__ a, float* __restrict__ b, int64_t pixels,
                            int c, int ctot, int c0, int dir) {
-    const int64_t total = pixels * c;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int ch = (int)(i % c);
-        const int64_t p = i / c;
-        if (dir == 0) b[p * ctot + c0 + ch] = a[i];
-        else if (dir == 1) b[i] = a[p * ctot + c0 + ch];
-        else b[i] += a[p * ctot + c0 + ch];
+    const uint32_t cv = (uint32_t)c / V;
+    for (int64_t p0 = (int64_t)blockIdx.x * 64; p0 < pixels; p0 += (int64_t)gridDim.x * 64) {
+        const uint32_t items = (uint32_t)(pixels - p0 < 64 ? pixels - p0 : 64) * cv;
+        for (uint32_t i = threadIdx.x; i < items; i += blockDim.x) {
+            const uint32_t p = i / cv, k = (i - p * cv) * V;
+            const int64_t thin = (p0 + p) * c + k, wide = (p0 + p) * ctot + c0 + k;
+            if (dir == 0) {
+                Vec<V>::ld(a + thin).st(b + wide);
+            } else {
+                Vec<V> v = Vec<V>::ld(a + wide);
+                if (dir != 1) {
+                    const Vec<V> o = Vec<V>::ld(b + thin);
+#pragma unroll
+                    for (int j = 0; j < V; j++) v.v[j] = o.v[j] + v.v[j];
+                }
+                v.st(b + thin);
+            }
+        }
     }
 }
 
@@ -559,6 +611,13 @@ int grid_for(int64_t total) {
     if (g > 8192) g = 8192;
     if (g < 1) g = 1;
     return (int)g;
+}
+
+// whether four-float accesses of arrays with these channel counts and the
+// first of them c0 are aligned
+bool vec4(const void* p, const void* q, int64_t c, int64_t ctot, int64_t c0) {
+    return ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(q)) & 15) == 0 &&
+           ((c | ctot | c0) & 3) == 0;
 }
 
 int status() { return hipGetLastError() == hipSuccess ? 0 : MPLBWS_ERR_HIP; }
@@ -659,23 +718,36 @@ int mplbws_pool2_bwd(const float* dout, float* din, int n, int h, int wd, int c)
 
 int mplbws_up2_fwd(const float* in, float* out, int n, int h, int wd, int c, int ctot, int c0) {
     if (!in || !out || c0 < 0 || c0 + c > ctot) return MPLBWS_ERR_ARG;
-    hipLaunchKernelGGL(k_up_fwd, dim3(grid_for((int64_t)n * 4 * h * wd * c)), dim3(256), 0, 0, in,
-                       out, n, h, wd, c, ctot, c0);
+    const int64_t rows = (int64_t)n * h;
+    const dim3 grd((unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, 65536)));
+    if (vec4(in, out, c, ctot, c0))
+        hipLaunchKernelGGL(k_up_fwd<4>, grd, dim3(256), 0, 0, in, out, rows, wd, c, ctot, c0);
+    else
+        hipLaunchKernelGGL(k_up_fwd<1>, grd, dim3(256), 0, 0, in, out, rows, wd, c, ctot, c0);
     return status();
 }
 
 int mplbws_up2_bwd(const float* dout, float* din, int n, int h, int wd, int c, int ctot, int c0) {
     if (!dout || !din || c0 < 0 || c0 + c > ctot) return MPLBWS_ERR_ARG;
-    hipLaunchKernelGGL(k_up_bwd, dim3(grid_for((int64_t)n * h * wd * c)), dim3(256), 0, 0, dout,
-                       din, n, h, wd, c, ctot, c0);
+    const int64_t rows = (int64_t)n * h;
+    const dim3 grd((unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, 65536)));
+    if (vec4(dout, din, c, ctot, c0))
+        hipLaunchKernelGGL(k_up_bwd<4>, grd, dim3(256), 0, 0, dout, din, rows, wd, c, ctot, c0);
+    else
+        hipLaunchKernelGGL(k_up_bwd<1>, grd, dim3(256), 0, 0, dout, din, rows, wd, c, ctot, c0);
     return status();
 }
 
 int mplbws_channels(const float* src, float* dst, int64_t pixels, int c, int ctot, int c0,
                     int direction) {
     if (!src || !dst || c0 < 0 || c0 + c > ctot) return MPLBWS_ERR_ARG;
-    hipLaunchKernelGGL(k_channels, dim3(grid_for(pixels * c)), dim3(256), 0, 0, src, dst, pixels,
-                       c, ctot, c0, direction);
+    const dim3 grd((unsigned)std::max<int64_t>(1, std::min<int64_t>((pixels + 63) / 64, 65536)));
+    if (vec4(src, dst, c, ctot, c0))
+        hipLaunchKernelGGL(k_channels<4>, grd, dim3(256), 0, 0, src, dst, pixels, c, ctot, c0,
+                           direction);
+    else
+        hipLaunchKernelGGL(k_channels<1>, grd, dim3(256), 0, 0, src, dst, pixels, c, ctot, c0,
+                           direction);
     return status();
 }
 
