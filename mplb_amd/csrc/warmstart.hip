@@ -1,7 +1,7 @@
 // warmstart.hip -- kernels of the learned warm start (a small U-Net that
 // predicts the steady cavity flow from the obstacle mask and Re): 3x3
 // convolutions as implicit GEMMs on the gfx950 matrix cores
-// (v_mfma_f32_32x32x8_bf16: BF16 operands, FP32 accumulation), their data
+// (v_mfma_f32_32x32x16_bf16: BF16 operands, FP32 accumulation), their data
 // and weight gradients, and the element-wise layers, loss and optimiser.
 // C ABI in include/mplbws.h.  No reference counterpart: the reference
 // starts every run from its initial macros.
@@ -15,10 +15,13 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 namespace {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWaves = 4;  // waves per workgroup
@@ -42,45 +45,50 @@ __device__ __forceinline__ uint2 to_bf16x4(const float4& f) {
 // Forward 3x3 convolution as an implicit GEMM, out[m][co] = sum_{tap, ci}
 // in[shift_tap(m)][ci] * w[tap][ci][co], zero padding at the image edges.
 //
-// A workgroup (4 waves) owns a tile of TP = 128 WM output pixels -- R whole
-// rows of W0 = min(wd, 128) columns -- and CG = 32 WN output channels.
-// Input channels go in chunks of kCC: the chunk's input tile with its
-// one-pixel halo is converted to BF16 once into LDS (zeros outside the
-// image), and so are the chunk's weights, in the MFMA operand layout; the
+// A workgroup (4 waves) owns a tile of TP = 128 WM output pixels -- R rows of
+// W0 <= 32 columns, nearly square so that its halo is small -- and CG = 32 WN
+// output channels.  Input channels go in chunks of kCC: the chunk's input tile
+// with its one-pixel halo is converted to BF16 once into LDS (zeros outside
+// the image), and so are the chunk's weights, in the MFMA operand layout; the
 // waves then run the 9 taps from LDS only.  Wave v takes pixels
 // [32 WM v, 32 WM (v + 1)) of the tile and all CG channels: WM x WN
-// accumulators of 32x32, each A fragment feeding WN of them and each B
-// fragment WM.  WM = 2 for large images (fewer, fuller workgroups), 1 where
-// that leaves too few workgroups; WN = 1 for layers of at most 32 output
-// channels.
+// accumulators of 32x32.  The weights are the A operand, so a lane's
+// accumulators hold four consecutive channels of one pixel, one 16-byte store.
 //
-// MFMA 32x32x8 (BF16 in, FP32 accumulate) lane layout: lane l holds
-// A[l%32][4(l/32) .. +3] and B[4(l/32) .. +3][l%32]; the accumulator
+// Bound: the staging, whose latency two to three workgroups per CU hide in
+// part: 32 images of 128 x 128, 72 to 24 channels read and write 201 MB, 32 us
+// of HBM, and take 62 us (135 with tiles of one row of 128 pixels, products of
+// 8 channels, integer rounding to BF16 and 64-bit addresses).  64 x 64, 48 to
+// 48 channels 51 -> 20 us, 128 to 64 channels at 128 x 128 266 -> 140 us.
+//
+// MFMA 32x32x16 (BF16 in, FP32 accumulate) lane layout: lane l holds
+// A[l%32][8(l/32) .. +7] and B[8(l/32) .. +7][l%32]; the accumulator
 // element 4i+j of lane l is C[8i + 4(l/32) + j][l%32].
 constexpr int kCC = 32;              // input channels per LDS chunk
-constexpr int kPixStride = kCC + 4;  // BF16 elements per staged pixel (the
-                                     // 8-byte pad spreads a wave's reads
+constexpr int kPixStride = kCC + 8;  // BF16 elements per staged pixel (the
+                                     // 16-byte pad spreads a wave's reads
                                      // over all LDS banks)
-constexpr int kMaxW0 = 128;
 
 struct ConvTile {
     int W0, R, tiles_x, tiles_y;
 };
 
+// pixels staged for a tile of tp pixels: the largest (R + 2)(W0 + 2)
+__host__ __device__ constexpr int conv_max_staged(int tp) { return tp == 256 ? 340 : 204; }
+
+// equal columns of at most 32, and as many rows as the tile's pixels and the
+// staged ones allow
 __host__ __device__ inline ConvTile conv_tile(int h, int wd, int tp) {
     ConvTile t;
-    t.W0 = wd < kMaxW0 ? wd : kMaxW0;
+    t.tiles_x = (wd + 31) / 32;
+    t.W0 = (wd + t.tiles_x - 1) / t.tiles_x;
     t.R = tp / t.W0;
-    if (t.R < 1) t.R = 1;
+    const int fit = conv_max_staged(tp) / (t.W0 + 2) - 2;
+    if (t.R > fit) t.R = fit;
     if (t.R > h) t.R = h;
-    t.tiles_x = (wd + t.W0 - 1) / t.W0;
     t.tiles_y = (h + t.R - 1) / t.R;
     return t;
 }
-
-// pixels staged for a tile of tp pixels: the largest (R + 2)(W0 + 2) over
-// the widths; the host refuses shapes above it
-__host__ __device__ constexpr int conv_max_staged(int tp) { return tp == 256 ? 520 : 390; }
 
 // q = e / d, r = e - q d for 0 <= e < 2^22 and 1 <= d <= 2^10 through a
 // float reciprocal (error below one unit before the correction)
@@ -98,175 +106,217 @@ __device__ __forceinline__ int fdiv(int e, const FastDiv& f, int* r) {
     return q;
 }
 
-template <int WM, int WN>
-__global__ __launch_bounds__(64 * kWaves) void k_conv_fwd(const float* __restrict__ in,
+// eight floats as BF16 (nearest even), one v_cvt_pk_bf16_f32 per pair
+__device__ __forceinline__ bf16x8 to_bf16x8(const float4& a, const float4& b) {
+    const f32x8 f = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    return __builtin_convertvector(f, bf16x8);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf(const float* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ float4 buf_ld4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+__device__ __forceinline__ float buf_ld1(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+}
+
+// workgroups are dealt to the 8 XCDs in turn: consecutive tiles, which share
+// their halos, on one of them
+__device__ __forceinline__ int tile_order(int i, int count) {
+    const int per = count / 8, whole = per * 8;
+    return i < whole ? (i % 8) * per + i / 8 : i;
+}
+
+// VEC: cout is a multiple of four, and w and out are aligned for 16-byte
+// accesses
+template <int WM, int WN, bool VEC>
+__global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const float* __restrict__ in,
                                                           const float* __restrict__ w,
                                                           const float* __restrict__ bias,
                                                           float* __restrict__ out, int n,
                                                           int h, int wd, int cin, int cout,
                                                           int relu) {
-    constexpr int TP = 128 * WM, CG = 32 * WN;
+    constexpr int TP = 128 * WM, CG = 32 * WN, NT = 64 * kWaves;
     __shared__ __attribute__((aligned(16))) short s_in[conv_max_staged(TP) * kPixStride];
-    // B fragments: [tap][kstep][g][co 0 .. CG-1][4]
-    __shared__ __attribute__((aligned(16))) short s_w[9 * (kCC / 8) * 2 * CG * 4];
+    // A fragments: [tap][8 input channels][co 0 .. CG-1][8]
+    __shared__ __attribute__((aligned(16))) short s_w[9 * (kCC / 8) * CG * 8];
     const ConvTile T = conv_tile(h, wd, TP);
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int row = lane & 31, g = lane >> 5;
     const int tiles = T.tiles_x * T.tiles_y;
-    const int pn = (int)blockIdx.x / tiles;
-    const int t = (int)blockIdx.x % tiles;
+    const int bid = tile_order((int)blockIdx.x, (int)gridDim.x);
+    const int pn = bid / tiles;
+    const int t = bid % tiles;
     const int y0 = (t / T.tiles_x) * T.R, x0 = (t % T.tiles_x) * T.W0;
     const int co0 = (int)blockIdx.y * CG;
-    const int SW = T.W0 + 2, SH = T.R + 2;
-    const FastDiv dW0 = fast_div(T.W0);
-    // this lane's A rows (pixels) in its WM pixel tiles; a lane past the
-    // tile reads pixel (0, 0) instead (its results are never stored)
-    int pbase[WM];
+    const int SW = T.W0 + 2, SP = (T.R + 2) * SW;
+    const FastDiv dW0 = fast_div(T.W0), dsw = fast_div(SW);
+    // this lane's pixel in its WM pixel tiles, and the first of the 3 x 3
+    // staged ones it reads; a lane past the tile reads those of pixel (0, 0)
+    // instead (its results are never stored)
+    int pbase[WM], px[WM], py[WM];
 #pragma unroll
     for (int mt = 0; mt < WM; mt++) {
         int tx;
         int ty = fdiv(wave * 32 * WM + mt * 32 + row, dW0, &tx);
+        px[mt] = x0 + tx;
+        py[mt] = ty < T.R ? y0 + ty : h;
         if (ty >= T.R) ty = tx = 0;
-        pbase[mt] = ((ty + 1) * SW + tx + 1) * kPixStride + 4 * g;
+        pbase[mt] = (ty * SW + tx) * kPixStride + 8 * g;
+    }
+    // Loads by buffer offsets that hold for every chunk, with the chunk and
+    // the weight row as scalar offsets and zeros (an offset past the end)
+    // outside the image and the weights: with 64-bit addresses and selects
+    // the staging issued three quarters of the kernel's instructions.
+    // Input item k: 8 channels of a staged pixel.
+    constexpr int kIn = (conv_max_staged(TP) * (kCC / 8) + NT - 1) / NT;
+    const int ya = y0 > 0 ? y0 - 1 : 0, yb = y0 + T.R + 1 < h ? y0 + T.R + 1 : h;
+    const uint32_t ibytes = (uint32_t)(yb - ya) * (uint32_t)wd * (uint32_t)cin * 4u;
+    const __amdgpu_buffer_rsrc_t rin = buf(in + ((int64_t)pn * h + ya) * wd * cin, ibytes);
+    const int c8 = (int)threadIdx.x & 3;
+    uint32_t ioff[kIn];
+#pragma unroll
+    for (int k = 0; k < kIn; k++) {
+        const int sp = ((int)threadIdx.x + k * NT) >> 2;
+        int sx;
+        const int sy = fdiv(sp, dsw, &sx);
+        const int yy = y0 + sy - 1, xx = x0 + sx - 1;
+        ioff[k] = sp < SP && yy >= 0 && yy < h && xx >= 0 && xx < wd
+                      ? ((uint32_t)((yy - ya) * wd + xx) * (uint32_t)cin + 8u * c8) * 4u
+                      : ibytes;
+    }
+    // Weight item k: 8 input channels of one tap by 4 output channels.
+    constexpr int kTot = 9 * (kCC / 8) * (CG / 4), kW = (kTot + NT - 1) / NT;
+    const uint32_t wbytes = 9u * (uint32_t)cin * (uint32_t)cout * 4u;
+    const __amdgpu_buffer_rsrc_t rw = buf(w, wbytes);
+    uint32_t woff[kW];
+#pragma unroll
+    for (int k = 0; k < kW; k++) {
+        const int e = (int)threadIdx.x + k * NT;
+        const int oc = co0 + (e % (CG / 4)) * 4, j = e / (CG / 4);
+        woff[k] = e < kTot && oc < cout
+                      ? (((uint32_t)(j >> 2) * cin + 8u * (j & 3)) * (uint32_t)cout + oc) * 4u
+                      : wbytes;
     }
     f32x16 acc[WM][WN] = {};
-    const float* img = in + (int64_t)pn * h * wd * cin;
     for (int c0 = 0; c0 < cin; c0 += kCC) {
         const int cc = cin - c0 < kCC ? cin - c0 : kCC;  // a multiple of 8
-        const int q8 = cc / 8;
-        __syncthreads();  // the previous chunk's reads are done
-        // input tile + halo in BF16, channels c0 .. c0 + cc: item e = one
-        // staged pixel's 8 channels (consecutive items: consecutive channel
-        // groups, then pixels); each thread issues the loads of kBatch
-        // items before converting any, so they are in flight together
-        {
-            const int total = SH * SW * q8;
-            const FastDiv dq8 = fast_div(q8), dsw = fast_div(SW);
-            constexpr int kBatch = 4;
-            for (int e0 = threadIdx.x; e0 < total; e0 += 64 * kWaves * kBatch) {
-                float4 f[kBatch][2];
-                int slot[kBatch];
+        const int g8 = (cc + 15) / 16 * 2;  // groups of 8 staged, zeros past cc
+        float4 f[kIn][2];
 #pragma unroll
-                for (int k = 0; k < kBatch; k++) {
-                    const int e = e0 + k * 64 * kWaves;
-                    f[k][0] = f[k][1] = float4{0.f, 0.f, 0.f, 0.f};
-                    slot[k] = -1;
-                    if (e < total) {
-                        int c8, sx;
-                        const int sp = fdiv(e, dq8, &c8);
-                        const int sy = fdiv(sp, dsw, &sx);
-                        const int yy = y0 + sy - 1, xx = x0 + sx - 1;
-                        slot[k] = sp * kPixStride + 8 * c8;
-                        if (yy >= 0 && yy < h && xx >= 0 && xx < wd) {
-                            const float* src = img + ((int64_t)yy * wd + xx) * cin + c0 + 8 * c8;
-                            f[k][0] = *reinterpret_cast<const float4*>(src);
-                            f[k][1] = *reinterpret_cast<const float4*>(src + 4);
-                        }
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < kBatch; k++) {
-                    if (slot[k] < 0) continue;
-                    *reinterpret_cast<uint2*>(&s_in[slot[k]]) = to_bf16x4(f[k][0]);
-                    *reinterpret_cast<uint2*>(&s_in[slot[k] + 4]) = to_bf16x4(f[k][1]);
-                }
-            }
+        for (int k = 0; k < kIn; k++) {
+            const uint32_t off = 8 * c8 < cc ? ioff[k] : ibytes;
+            f[k][0] = buf_ld4(rin, off, c0 * 4u);
+            f[k][1] = buf_ld4(rin, off, c0 * 4u + 16u);
         }
-        // weights of the chunk in B-fragment order, zero past cout: thread
-        // -> four output channels co4 .. co4 + 3 (one 16-byte load when
-        // they lie inside cout and cout is a multiple of 4) and the (tap,
-        // ci) pairs j = tid / (CG / 4) + k (256 / (CG / 4)); every load of
-        // the chunk is issued before any is converted, so they are in
-        // flight together
-        {
-            constexpr int groups = CG / 4;
-            constexpr int step = 64 * kWaves / groups;
-            constexpr int kMax = (9 * kCC + step - 1) / step;  // loads per thread
-            const int co4 = ((int)threadIdx.x % groups) * 4;
-            const int oc = co0 + co4;
-            const int pairs = 9 * cc;
-            const int j0 = (int)threadIdx.x / groups;
-            const FastDiv dcc = fast_div(cc);
-            const bool vec = (cout & 3) == 0 && oc + 3 < cout;
-            float4 v[kMax];
+        float4 u[8];
+        auto load_w = [&](int k) {
+            const int j = ((int)threadIdx.x + k * NT) / (CG / 4);
+            const uint32_t off = 8 * (j & 3) < cc ? woff[k] : wbytes;
 #pragma unroll
-            for (int k = 0; k < kMax; k++) {
-                const int j = j0 + k * step;
-                v[k] = float4{0.f, 0.f, 0.f, 0.f};
-                if (j < pairs && oc < cout) {
-                    int ci;
-                    const int tap = fdiv(j, dcc, &ci);
-                    const float* src = w + ((int64_t)tap * cin + c0 + ci) * cout + oc;
-                    if (vec) {
-                        v[k] = *reinterpret_cast<const float4*>(src);
-                    } else {
-                        v[k].x = src[0];
-                        if (oc + 1 < cout) v[k].y = src[1];
-                        if (oc + 2 < cout) v[k].z = src[2];
-                        if (oc + 3 < cout) v[k].w = src[3];
-                    }
+            for (int r = 0; r < 8; r++) {
+                const uint32_t so = (uint32_t)(c0 + r) * (uint32_t)cout * 4u;
+                if constexpr (VEC) {
+                    u[r] = buf_ld4(rw, off, so);
+                } else {
+                    const int left = off < wbytes ? cout - (int)((off / 4u) % (uint32_t)cout) : 0;
+                    u[r].x = buf_ld1(rw, off, so);
+                    u[r].y = buf_ld1(rw, left > 1 ? off + 4u : wbytes, so);
+                    u[r].z = buf_ld1(rw, left > 2 ? off + 8u : wbytes, so);
+                    u[r].w = buf_ld1(rw, left > 3 ? off + 12u : wbytes, so);
                 }
             }
+        };
+        load_w(0);
+        if (c0) __syncthreads();  // the previous chunk's reads are done
 #pragma unroll
-            for (int k = 0; k < kMax; k++) {
-                const int j = j0 + k * step;
-                if (j >= pairs) break;
-                int ci;
-                const int tap = fdiv(j, dcc, &ci);
-                const int ks = ci >> 3, gg = (ci >> 2) & 1, tt = ci & 3;
-                short* dst = &s_w[((((tap * (kCC / 8) + ks) * 2 + gg) * CG) + co4) * 4 + tt];
-                dst[0] = to_bf16(v[k].x);
-                dst[4] = to_bf16(v[k].y);
-                dst[8] = to_bf16(v[k].z);
-                dst[12] = to_bf16(v[k].w);
-            }
+        for (int k = 0; k < kIn; k++) {
+            const int sp = ((int)threadIdx.x + k * NT) >> 2;
+            if (sp < SP && c8 < g8)
+                *reinterpret_cast<bf16x8*>(&s_in[sp * kPixStride + 8 * c8]) =
+                    to_bf16x8(f[k][0], f[k][1]);
+        }
+#pragma unroll
+        for (int k = 0; k < kW; k++) {
+            if (k) load_w(k);
+            const int e = (int)threadIdx.x + k * NT;
+            const int co4 = (e % (CG / 4)) * 4, j = e / (CG / 4);
+            if (e >= kTot || (j & 3) >= g8) continue;
+            short* dst = &s_w[(j * CG + co4) * 8];
+            auto put = [&](int c, float4 a, float4 b) {
+                *reinterpret_cast<bf16x8*>(dst + 8 * c) = to_bf16x8(a, b);
+            };
+            put(0, float4{u[0].x, u[1].x, u[2].x, u[3].x}, float4{u[4].x, u[5].x, u[6].x, u[7].x});
+            put(1, float4{u[0].y, u[1].y, u[2].y, u[3].y}, float4{u[4].y, u[5].y, u[6].y, u[7].y});
+            put(2, float4{u[0].z, u[1].z, u[2].z, u[3].z}, float4{u[4].z, u[5].z, u[6].z, u[7].z});
+            put(3, float4{u[0].w, u[1].w, u[2].w, u[3].w}, float4{u[4].w, u[5].w, u[6].w, u[7].w});
         }
         __syncthreads();
-        for (int tap = 0; tap < 9; tap++) {
-            const int shift = ((tap / 3 - 1) * SW + (tap % 3 - 1)) * kPixStride;
-            for (int ks = 0; ks < q8; ks++) {
-                bf16x4 a[WM], b[WN];
+        // the taps' offsets are immediate ones but for the row's
+        auto products = [&](auto steps) {
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                const short* rows[WM];
 #pragma unroll
                 for (int mt = 0; mt < WM; mt++)
-                    a[mt] = *reinterpret_cast<const bf16x4*>(&s_in[pbase[mt] + shift + ks * 8]);
+                    rows[mt] = &s_in[pbase[mt] + dy * SW * kPixStride];
+                const short* wl = &s_w[(g * CG + row) * 8];
 #pragma unroll
-                for (int nt = 0; nt < WN; nt++)
-                    b[nt] = *reinterpret_cast<const bf16x4*>(
-                        &s_w[((((tap * (kCC / 8) + ks) * 2 + g) * CG) + nt * 32 + row) * 4]);
+                for (int dx = 0; dx < 3; dx++)
 #pragma unroll
-                for (int mt = 0; mt < WM; mt++)
+                    for (int ks = 0; ks < decltype(steps)::value; ks++) {
+                        bf16x8 a[WN], b[WM];
 #pragma unroll
-                    for (int nt = 0; nt < WN; nt++)
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a[mt], b[nt],
-                                                                                acc[mt][nt], 0, 0, 0);
+                        for (int mt = 0; mt < WM; mt++)
+                            b[mt] = *reinterpret_cast<const bf16x8*>(rows[mt] + dx * kPixStride +
+                                                                     ks * 16);
+#pragma unroll
+                        for (int nt = 0; nt < WN; nt++)
+                            a[nt] = *reinterpret_cast<const bf16x8*>(
+                                wl + (((3 * dy + dx) * (kCC / 8) + 2 * ks) * CG + nt * 32) * 8);
+#pragma unroll
+                        for (int mt = 0; mt < WM; mt++)
+#pragma unroll
+                            for (int nt = 0; nt < WN; nt++)
+                                acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                    a[nt], b[mt], acc[mt][nt], 0, 0, 0);
+                    }
             }
-        }
+        };
+        if (g8 == 4) products(std::integral_constant<int, 2>{});
+        else products(std::integral_constant<int, 1>{});
     }
-    // epilogue: bias, relu, FP32 store (32 consecutive channels per row)
+    // epilogue: bias, relu, FP32 store
 #pragma unroll
-    for (int nt = 0; nt < WN; nt++) {
-        const int co = co0 + nt * 32 + row;
-        if (co >= cout) continue;
-        const float bv = bias ? bias[co] : 0.f;
+    for (int nt = 0; nt < WN; nt++)
 #pragma unroll
-        for (int mt = 0; mt < WM; mt++)
+        for (int i = 0; i < 4; i++) {
+            const int co = co0 + nt * 32 + 8 * i + 4 * g;
+            float bv[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                int tx1;
-                const int p1 = wave * 32 * WM + mt * 32 + 8 * i + 4 * g;
-                const int ty1 = fdiv(p1, dW0, &tx1);
+            for (int j = 0; j < 4; j++) bv[j] = bias && co + j < cout ? bias[co + j] : 0.f;
+#pragma unroll
+            for (int mt = 0; mt < WM; mt++) {
+                if (py[mt] >= h || px[mt] >= wd || co >= cout) continue;
+                float v[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    int tx = tx1 + j, ty = ty1;
-                    if (tx >= T.W0) ty = fdiv(p1 + j, dW0, &tx);
-                    if (ty >= T.R || y0 + ty >= h || x0 + tx >= wd) continue;
-                    float v = acc[mt][nt][4 * i + j] + bv;
-                    if (relu) v = v > 0.f ? v : 0.f;
-                    out[(((int64_t)pn * h + y0 + ty) * wd + x0 + tx) * cout + co] = v;
+                    v[j] = acc[mt][nt][4 * i + j] + bv[j];
+                    if (relu) v[j] = v[j] > 0.f ? v[j] : 0.f;
+                }
+                float* dst = out + (((int64_t)pn * h + py[mt]) * wd + px[mt]) * cout + co;
+                if constexpr (VEC) {
+                    *reinterpret_cast<float4*>(dst) = float4{v[0], v[1], v[2], v[3]};
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (co + j < cout) dst[j] = v[j];
                 }
             }
-    }
+        }
 }
 
 // weights of the data gradient: wt[tap][co][ci] = w[8 - tap][ci][co]
@@ -631,32 +681,32 @@ int mplbws_conv3x3_fwd(const float* in, const float* w, const float* bias, float
     if (!in || !w || !out || n <= 0 || h <= 0 || wd <= 0 || cin <= 0 || cout <= 0 ||
         cin % 8 != 0)
         return MPLBWS_ERR_ARG;
-    // WM = 2 (256-pixel tiles) unless that gives fewer than 1024
-    // workgroups; WN = 1 for at most 32 output channels
+    // WN = 1 for at most 32 output channels; WM = 2 (256-pixel tiles) while
+    // that gives every CU two workgroups (64 x 64 x 48, 32 images: 512 of
+    // them and 22.6 us, 28.8 with WM = 1; 128 or fewer: the same within 0.3 us)
     const int wn = cout > 32 ? 2 : 1;
     const int64_t groups = (cout + 32 * wn - 1) / (32 * wn);
     const ConvTile T2 = conv_tile(h, wd, 256);
-    const int wm = (int64_t)n * T2.tiles_x * T2.tiles_y * groups >= 1024 &&
-                           (T2.R + 2) * (T2.W0 + 2) <= conv_max_staged(256)
-                       ? 2
-                       : 1;
+    const int wm = (int64_t)n * T2.tiles_x * T2.tiles_y * groups >= 512 ? 2 : 1;
     const ConvTile T = conv_tile(h, wd, 128 * wm);
     const int64_t wgs = (int64_t)n * T.tiles_x * T.tiles_y;
-    if (wgs >= ((int64_t)1 << 31) || (T.R + 2) * (T.W0 + 2) > conv_max_staged(128 * wm))
+    // (a tile's rows and the weights are addressed by 32-bit offsets)
+    if (wgs >= ((int64_t)1 << 31) || (int64_t)(T.R + 2) * wd * cin >= (int64_t)1 << 29 ||
+        9LL * cin * cout >= (int64_t)1 << 29)
         return MPLBWS_ERR_ARG;
     const dim3 grd((unsigned)wgs, (unsigned)groups), blk(64 * kWaves);
-    if (wm == 2 && wn == 2)
-        hipLaunchKernelGGL((k_conv_fwd<2, 2>), grd, blk, 0, 0, in, w, bias, out, n, h, wd, cin,
-                           cout, relu);
-    else if (wm == 2)
-        hipLaunchKernelGGL((k_conv_fwd<2, 1>), grd, blk, 0, 0, in, w, bias, out, n, h, wd, cin,
-                           cout, relu);
-    else if (wn == 2)
-        hipLaunchKernelGGL((k_conv_fwd<1, 2>), grd, blk, 0, 0, in, w, bias, out, n, h, wd, cin,
-                           cout, relu);
-    else
-        hipLaunchKernelGGL((k_conv_fwd<1, 1>), grd, blk, 0, 0, in, w, bias, out, n, h, wd, cin,
-                           cout, relu);
+    const bool vec = vec4(w, out, cout, 0, 0);
+#define X(WM, WN)                                                                             \
+    if (wm == WM && wn == WN) {                                                               \
+        if (vec)                                                                              \
+            hipLaunchKernelGGL((k_conv_fwd<WM, WN, true>), grd, blk, 0, 0, in, w, bias, out, n, \
+                               h, wd, cin, cout, relu);                                       \
+        else                                                                                  \
+            hipLaunchKernelGGL((k_conv_fwd<WM, WN, false>), grd, blk, 0, 0, in, w, bias, out, n, \
+                               h, wd, cin, cout, relu);                                       \
+    }
+    X(2, 2) X(2, 1) X(1, 2) X(1, 1)
+#undef X
     return status();
 }
 

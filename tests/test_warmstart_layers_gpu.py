@@ -1,11 +1,13 @@
 """The warm-start network's layers at the edges of their kernels' tiles and
-vector widths: upsampling and channel copies exactly."""
+vector widths: upsampling and channel copies exactly, convolutions against the
+CPU layer oracle (BF16 operands, float64 sums)."""
 import sys
 
 import numpy as np
 import pytest
 
 from mplb_amd import warmstart as ws
+from oracle import nn_oracle as nno
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +52,31 @@ def test_upsampling_and_channel_copies(n, h, wd, c, ctot, c0):
     ref = fine.copy()
     ref[..., c0:c0 + c] = thin
     assert np.array_equal(df.numpy(), ref)
+
+
+# (n, h, w, cin, cout): one pixel, tiles of 32 columns and their edges, rows
+# past a tile, chunks of 32 input channels with remainders of 8 and 16, 4-, 1-
+# and 3-channel remainders of the output, the larger tiles' smallest grid
+CONV = [(1, 1, 1, 8, 4), (2, 3, 2, 8, 1), (1, 5, 33, 24, 24), (3, 32, 32, 40, 36),
+        (1, 17, 65, 48, 33), (2, 40, 31, 72, 64), (1, 9, 100, 56, 67), (33, 64, 64, 8, 8),
+        (1, 70, 7, 16, 32)]
+
+
+@pytest.mark.parametrize("n,h,wd,cin,cout", CONV)
+def test_convolution_forward(n, h, wd, cin, cout):
+    log("conv %s" % ((n, h, wd, cin, cout),))
+    lib, rng = ws.load(), np.random.default_rng(7)
+    A = ws.DeviceArray.from_numpy
+    x = rng.standard_normal((n, h, wd, cin)).astype(np.float32)
+    w = (rng.standard_normal((9, cin, cout)) / 8).astype(np.float32)
+    b = rng.standard_normal(cout).astype(np.float32)
+    dx, dw, db, out = A(x), A(w), A(b), ws.DeviceArray((n, h, wd, cout))
+    mag = nno.conv3x3(np.abs(x), np.abs(w)) + np.abs(b)
+    for bias, relu in ((True, 1), (False, 0)):
+        ck(lib.mplbws_conv3x3_fwd(dx.p, dw.p, db.p if bias else None, out.p, n, h, wd, cin, cout,
+                                  relu))
+        ref = nno.conv3x3(x, w, b if bias else None, relu=bool(relu))
+        # FP32 sums of 9 cin exact products and the bias: at most that many
+        # roundings of partial sums bounded by the sum of magnitudes
+        tol = (9 * cin + 1) * 2.0 ** -24 * mag
+        assert (np.abs(out.numpy() - ref) <= tol).all()
