@@ -19,28 +19,13 @@
 
 namespace {
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWaves = 4;  // waves per workgroup
-
-// FP32 -> BF16, round to nearest even (finite inputs), in integer
-// arithmetic: measured faster here than the packed hardware conversion
-// (v_cvt_pk_bf16_f32) in these staging loops
-__device__ __forceinline__ short to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (short)(u >> 16);
-}
-// two at once, a in the low half
-__device__ __forceinline__ uint32_t to_bf16x2(float a, float b) {
-    return (uint32_t)(uint16_t)to_bf16(a) | ((uint32_t)(uint16_t)to_bf16(b) << 16);
-}
-__device__ __forceinline__ uint2 to_bf16x4(const float4& f) {
-    return uint2{to_bf16x2(f.x, f.y), to_bf16x2(f.z, f.w)};
-}
 
 // Forward 3x3 convolution as an implicit GEMM, out[m][co] = sum_{tap, ci}
 // in[shift_tap(m)][ci] * w[tap][ci][co], zero padding at the image edges.
@@ -342,99 +327,259 @@ __host__ __device__ inline int wgrad_rows(int h, int wd) {
     return r;
 }
 
-// Weight gradient partials of one chunk: a wave computes a 32 (rows k =
-// tap*cin + ci) x 32 (co) tile of sum_m A[m][k] dout[m][co] over the
-// chunk's pixels, 8 per product (MFMA reduction dimension = pixels); the
-// waves take the chunk's rows in turn and their tiles are summed through
-// LDS in wave order.  partial[chunk][k][co].  The workgroups of the first
-// k tile also sum the dout values they load (FP32, fixed order) into the
-// bias-gradient partial bpart[chunk][co] when bpart is given.
-__global__ __launch_bounds__(64 * kWaves) void k_conv_wgrad(const float* __restrict__ in,
-                                                            const float* __restrict__ dout,
-                                                            float* __restrict__ partial,
-                                                            float* __restrict__ bpart,
-                                                            int h, int wd, int cin, int cout,
-                                                            int rows) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int K = 9 * cin;
-    const int k0 = blockIdx.x * 32, co0 = blockIdx.y * 32;
+// Weight gradient partials of one chunk of whole rows: partial[chunk][tap][ci]
+// [co] = sum over its pixels m of in[shift_tap(m)][ci] dout[m][co], products
+// of 16 pixels.  A workgroup takes 32 input and 32 output channels, one wave
+// per tap; sub-tiles of at most kGPix pixels (RT rows of SEG columns, a
+// multiple of 16) of dout, and of the input with a pixel around them, are
+// converted to BF16 once into LDS as they lie in HBM, a pixel's 32 channels in
+// a row, and read transposed (ds_read_b64_tr_b16): the product's reduction
+// runs over pixels, and a tap is a shift by whole pixels, which needs no
+// alignment.  The workgroups of the first input channels also sum the dout
+// values they load (FP32, fixed order) into bpart[chunk][co] when it is given.
+//
+// Bound: the loads of one sub-tile per workgroup in flight, and too few
+// workgroups for the chip when the chunks are few (one image of 64 x 64: 2 us
+// per sub-tile either way).  With both sums, us: 32 images of 64 x 64, 48 to 48
+// channels 123 -> 47, 128 x 128, 72 to 24 356 -> 100 and 128 to 64 731 -> 204,
+// 8 x 8, 128 to 64 18.7 -> 13.3 (before: every operand by 4-byte loads from
+// HBM, again for each of the 9 cin / 32 tiles, one wave's rows at a time).  A
+// workgroup per row of taps with the pixels dealt to 4 or 8 waves and their
+// tiles summed in LDS took 52 to 103, its staging three times as much.
+constexpr int kGWaves = 9;
+constexpr int kGPix = 256;   // pixels of dout staged
+constexpr int kGIn = 396;    // and of the input: (RT + 2)(SEG + 2), 4 rows of 64 the most
+
+// columns and rows of a sub-tile
+struct GradTile {
+    int seg, segs, rt;
+};
+__host__ __device__ inline GradTile grad_tile(int wd) {
+    GradTile t;
+    t.segs = (wd + 63) / 64;
+    t.seg = ((wd + t.segs - 1) / t.segs + 15) / 16 * 16;
+    t.rt = kGPix / t.seg;
+    return t;
+}
+
+// four pixels of one channel: the 16 lanes of a row each point at 4 channels
+// of one of them
+__device__ __forceinline__ s16x4 lds_tr(const short* p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+}
+
+// 8 channels at a byte offset, `left` of them (a multiple of 4 if VEC) real;
+// zeros past them and for off = bytes
+template <bool VEC>
+__device__ __forceinline__ void load8(float4* f, __amdgpu_buffer_rsrc_t r, uint32_t off, int left,
+                                      uint32_t bytes) {
+    if constexpr (VEC) {
+        f[0] = buf_ld4(r, left > 0 ? off : bytes, 0);
+        f[1] = buf_ld4(r, left > 4 ? off + 16u : bytes, 0);
+    } else {
+        float v[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) v[c] = buf_ld1(r, left > c ? off + 4u * c : bytes, 0);
+        f[0] = float4{v[0], v[1], v[2], v[3]};
+        f[1] = float4{v[4], v[5], v[6], v[7]};
+    }
+}
+
+// VEC: cin and cout are multiples of four, in and dout aligned for 16-byte
+// accesses
+template <bool VEC>
+__global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __restrict__ in,
+                                                                const float* __restrict__ dout,
+                                                                float* __restrict__ partial,
+                                                                float* __restrict__ bpart, int h,
+                                                                int wd, int cin, int cout,
+                                                                int rows) {
+    constexpr int NT = 64 * kGWaves, NP = NT / 4;
+    // [pixel][32 channels]
+    __shared__ __attribute__((aligned(16))) short s_x[kGIn * 32];
+    __shared__ __attribute__((aligned(16))) short s_d[kGPix * 32];
+    const GradTile T = grad_tile(wd);
+    const int lane = threadIdx.x & 63, tap = threadIdx.x >> 6;
+    const int ci0 = (int)blockIdx.x * 32, co0 = (int)blockIdx.y * 32;
     const int per_image = (h + rows - 1) / rows;
     const int pn = (int)blockIdx.z / per_image;
     const int r0 = ((int)blockIdx.z % per_image) * rows;
     const int r1 = r0 + rows < h ? r0 + rows : h;
-    const int row = lane & 31, g = lane >> 5;
-    const int k = k0 + row;  // A row of this lane
-    const bool kvalid = k < K;
-    const int tap = kvalid ? k / cin : 0, ci = kvalid ? k % cin : 0;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int co = co0 + row;  // B column of this lane
-    const bool cvalid = co < cout;
-    const float* inb = in + (int64_t)pn * h * wd * cin;
-    const float* db = dout + (int64_t)pn * h * wd * cout;
+    // the chunk's rows of dout, and of the input with one around
+    const int ya = r0 > 0 ? r0 - 1 : 0, yb = r1 < h ? r1 + 1 : h;
+    const uint32_t xbytes = (uint32_t)(yb - ya) * (uint32_t)wd * (uint32_t)cin * 4u;
+    const uint32_t dbytes = (uint32_t)(r1 - r0) * (uint32_t)wd * (uint32_t)cout * 4u;
+    const __amdgpu_buffer_rsrc_t rx = buf(in + ((int64_t)pn * h + ya) * wd * cin, xbytes);
+    const __amdgpu_buffer_rsrc_t rd = buf(dout + ((int64_t)pn * h + r0) * wd * cout, dbytes);
+    const int xw = T.seg + 2;
+    const FastDiv dseg = fast_div(T.seg), dxw = fast_div(xw);
+    // staging items: 8 channels of a pixel; a thread keeps its channels
+    constexpr int kX = (kGIn + NP - 1) / NP, kD = (kGPix + NP - 1) / NP;
+    const int c8 = (int)threadIdx.x % 4 * 8, p0 = (int)threadIdx.x / 4;
+    const int xleft = cin - ci0 - c8, dleft = cout - co0 - c8;
+    // the items' pixels in a sub-tile (rows past it: none), and their byte
+    // offsets from its first one
+    int xty[kX], xtx[kX], dty[kD], dtx[kD];
+    uint32_t xrel[kX], drel[kD];
+#pragma unroll
+    for (int k = 0; k < kX; k++) {
+        xty[k] = fdiv(p0 + k * NP, dxw, &xtx[k]) - 1;
+        xtx[k]--;
+        xrel[k] = ((uint32_t)(xty[k] * wd + xtx[k]) * (uint32_t)cin + ci0 + c8) * 4u;
+        if (xty[k] > T.rt) xty[k] = 1 << 30;
+    }
+#pragma unroll
+    for (int k = 0; k < kD; k++) {
+        dty[k] = fdiv(p0 + k * NP, dseg, &dtx[k]);
+        drel[k] = ((uint32_t)(dty[k] * wd + dtx[k]) * (uint32_t)cout + co0 + c8) * 4u;
+        if (dty[k] >= T.rt) dty[k] = 1 << 30;
+    }
+    float4 fx[kX][2], fd[kD][2];
+    // sub-tile: rows from ry, columns from cx
+    auto load = [&](int ry, int cx) {
+        const uint32_t xb = (uint32_t)((ry - ya) * wd + cx) * (uint32_t)cin * 4u;
+        const uint32_t db = (uint32_t)((ry - r0) * wd + cx) * (uint32_t)cout * 4u;
+#pragma unroll
+        for (int k = 0; k < kX; k++) {
+            const bool on = (uint32_t)(xty[k] + ry - ya) < (uint32_t)(yb - ya) &&
+                            (uint32_t)(xtx[k] + cx) < (uint32_t)wd;
+            load8<VEC>(fx[k], rx, xrel[k] + xb, on ? xleft : 0, xbytes);
+        }
+#pragma unroll
+        for (int k = 0; k < kD; k++) {
+            const bool on = dty[k] + ry < r1 && dtx[k] + cx < wd;
+            load8<VEC>(fd[k], rd, drel[k] + db, on ? dleft : 0, dbytes);
+        }
+    };
+    // this lane's part of a transposed read: group l / 16 reads channels
+    // 16 (l / 16 % 2) .. and pixels 8 (l / 32) .. of a product's 16
+    const int tr = (8 * (lane >> 5) + (lane & 15) / 4) * 32 + 16 * (lane >> 4 & 1) + 4 * (lane & 3);
+    const int shift = (tap / 3 * xw + tap % 3) * 32;
     f32x16 acc = {};
-    float bsum = 0.f;
-    for (int py = r0 + wave; py < r1; py += kWaves) {
-        const int yy = py + dy;
-        const bool yin = kvalid && yy >= 0 && yy < h;
-        for (int x0 = 0; x0 < wd; x0 += 8) {
-            bf16x4 a, b;
+    float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    load(r0, 0);
+    for (int ry = r0, cx = 0; ry < r1;) {
+        const int nx = cx + T.seg < wd ? cx + T.seg : 0, ny = nx ? ry : ry + T.rt;
+        if (ry > r0 || cx) __syncthreads();  // the products before have read
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int px = x0 + 4 * g + t;
-                const int xx = px + dx;
-                float av = 0.f, bv = 0.f;
-                if (px < wd) {
-                    if (yin && xx >= 0 && xx < wd) av = inb[((int64_t)yy * wd + xx) * cin + ci];
-                    if (cvalid) bv = db[((int64_t)py * wd + px) * cout + co];
-                }
-                bsum += bv;
-                a[t] = to_bf16(av);
-                b[t] = to_bf16(bv);
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
+        for (int k = 0; k < kX; k++)
+            if (p0 + k * NP < kGIn)
+                *reinterpret_cast<bf16x8*>(&s_x[(p0 + k * NP) * 32 + c8]) =
+                    to_bf16x8(fx[k][0], fx[k][1]);
+#pragma unroll
+        for (int k = 0; k < kD; k++) {
+            if (p0 + k * NP < kGPix)
+                *reinterpret_cast<bf16x8*>(&s_d[(p0 + k * NP) * 32 + c8]) =
+                    to_bf16x8(fd[k][0], fd[k][1]);
+            const float v[8] = {fd[k][0].x, fd[k][0].y, fd[k][0].z, fd[k][0].w,
+                                fd[k][1].x, fd[k][1].y, fd[k][1].z, fd[k][1].w};
+#pragma unroll
+            for (int c = 0; c < 8; c++) bsum[c] += v[c];
         }
-    }
-    __shared__ float bred[kWaves][2][32];
-    if (bpart && blockIdx.x == 0) {
-        bred[wave][g][row] = bsum;
         __syncthreads();
-        if (threadIdx.x < 32 && co0 + (int)threadIdx.x < cout) {
-            float s = 0.f;
-            for (int v = 0; v < kWaves; v++) s += bred[v][0][threadIdx.x] + bred[v][1][threadIdx.x];
-            bpart[(int64_t)blockIdx.z * cout + co0 + threadIdx.x] = s;
+        if (ny < r1) load(ny, nx);
+        const int nrows = r1 - ry < T.rt ? r1 - ry : T.rt;
+        // N products of a row, their reads ahead of them
+        auto products = [&](auto steps, const short* d, const short* x, int px) {
+            constexpr int N = decltype(steps)::value;
+            s16x8 a[N], b[N];
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                b[i] = __builtin_shufflevector(lds_tr(d + (px + 16 * i) * 32),
+                                               lds_tr(d + (px + 16 * i + 4) * 32), 0, 1, 2, 3, 4, 5,
+                                               6, 7);
+                a[i] = __builtin_shufflevector(lds_tr(x + (px + 16 * i) * 32),
+                                               lds_tr(x + (px + 16 * i + 4) * 32), 0, 1, 2, 3, 4, 5,
+                                               6, 7);
+            }
+            // pixels past the row's end: their dout is zero, and so has to be
+            // the input beside it, whatever it holds
+            if (wd - cx - px < 16 * N) {
+#pragma unroll
+                for (int i = 0; i < N; i++)
+#pragma unroll
+                    for (int t = 0; t < 8; t++)
+                        a[i][t] =
+                            px + 16 * i + 8 * (lane >> 5) + t < wd - cx ? a[i][t] : (short)0;
+            }
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[i]),
+                                                              __builtin_bit_cast(bf16x8, b[i]), acc,
+                                                              0, 0, 0);
+        };
+        for (int ty = 0; ty < nrows; ty++) {
+            const short* d = &s_d[ty * T.seg * 32 + tr];
+            const short* x = &s_x[ty * xw * 32 + tr + shift];
+            int px = 0;
+            for (; px + 64 <= T.seg; px += 64) products(std::integral_constant<int, 4>{}, d, x, px);
+            for (; px < T.seg; px += 16) products(std::integral_constant<int, 1>{}, d, x, px);
         }
+        ry = ny;
+        cx = nx;
     }
-    // sum the waves' tiles through LDS, then write this chunk's partial
-    __shared__ float red[kWaves][32][33];
+    const int row = lane & 31, g = lane >> 5;
+    if (co0 + row < cout) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) red[wave][8 * i + 4 * g + j][row] = acc[4 * i + j];
-    __syncthreads();
-    for (int e = threadIdx.x; e < 32 * 32; e += 64 * kWaves) {
-        const int r = e / 32, cc = e % 32;
+            for (int j = 0; j < 4; j++) {
+                const int ci = ci0 + 8 * i + 4 * g + j;
+                if (ci < cin)
+                    partial[(((int64_t)blockIdx.z * 9 + tap) * cin + ci) * cout + co0 + row] =
+                        acc[4 * i + j];
+            }
+    }
+    if (bpart && blockIdx.x == 0) {
+        __syncthreads();
+        float* red = reinterpret_cast<float*>(s_x);  // [thread / 4][channel]
+        static_assert(sizeof(float) * NT * 8 <= sizeof(s_x), "bias sums");
+#pragma unroll
+        for (int c = 0; c < 8; c++) red[threadIdx.x * 8 + c] = bsum[c];
+        __syncthreads();
+        // 16 threads per channel, then one
+        const int c = (int)threadIdx.x & 31, v0 = (int)threadIdx.x >> 5;
         float s = 0.f;
-        for (int v = 0; v < kWaves; v++) s += red[v][r][cc];
-        const int kk = k0 + r, oc = co0 + cc;
-        if (kk < K && oc < cout) partial[((int64_t)blockIdx.z * K + kk) * cout + oc] = s;
+        if (v0 < 16)
+            for (int v = v0; v < NP; v += 16) s += red[v * 32 + c];
+        __syncthreads();
+        if (v0 < 16) red[v0 * 32 + c] = s;
+        __syncthreads();
+        if (threadIdx.x < 32 && co0 + c < cout) {
+            s = 0.f;
+            for (int v = 0; v < 16; v++) s += red[v * 32 + c];
+            bpart[(int64_t)blockIdx.z * cout + co0 + c] = s;
+        }
     }
 }
 
-// dw = sum over chunks (chunk order: deterministic)
-// dst[i] = sum over the chunks of partial[c][i]: a workgroup takes 64
-// consecutive i, its four waves the chunks c = w, w + 4, ... (so each wave
-// has a quarter of the dependent adds), and the waves' sums are added in
-// wave order through LDS: a fixed order, reproducible sums.
+// dst[i] = sum over the chunks of partial[c][i], and the same of the bias
+// partials in the workgroups after those of dst (bdst: none if 0): a workgroup
+// takes 64 consecutive i, its four waves the chunks c = w, w + 4, ... (so each
+// wave has a quarter of the dependent adds, eight loads in flight), and the
+// waves' sums are added in wave order through LDS: a fixed order, reproducible
+// sums.
 constexpr int kSumWaves = 4;
 __global__ __launch_bounds__(64 * kSumWaves) void k_sum_partials(const float* __restrict__ partial,
                                                                  float* __restrict__ dst,
-                                                                 int64_t count, int nchunks) {
+                                                                 int64_t count,
+                                                                 const float* __restrict__ bpart,
+                                                                 float* __restrict__ bdst,
+                                                                 int64_t bcount, int nchunks) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+    int64_t i = (int64_t)blockIdx.x * 64 + lane;
+    const int64_t whole = (count + 63) / 64;
+    if (blockIdx.x >= whole) {
+        i -= whole * 64;
+        partial = bpart;
+        dst = bdst;
+        count = bcount;
+    }
     float s = 0.f;
-    if (i < count)
+    if (i < count) {
+#pragma unroll 8
         for (int c = w; c < nchunks; c += kSumWaves) s += partial[(int64_t)c * count + i];
+    }
     __shared__ float red[kSumWaves][64];
     red[w][lane] = s;
     __syncthreads();
@@ -691,8 +836,8 @@ int mplbws_conv3x3_fwd(const float* in, const float* w, const float* bias, float
     const ConvTile T = conv_tile(h, wd, 128 * wm);
     const int64_t wgs = (int64_t)n * T.tiles_x * T.tiles_y;
     // (a tile's rows and the weights are addressed by 32-bit offsets)
-    if (wgs >= ((int64_t)1 << 31) || (int64_t)(T.R + 2) * wd * cin >= (int64_t)1 << 29 ||
-        9LL * cin * cout >= (int64_t)1 << 29)
+    if (wgs >= ((int64_t)1 << 31) || (int64_t)(T.R + 2) * wd * cin >= (int64_t)1 << 30 ||
+        9LL * cin * cout >= (int64_t)1 << 30)
         return MPLBWS_ERR_ARG;
     const dim3 grd((unsigned)wgs, (unsigned)groups), blk(64 * kWaves);
     const bool vec = vec4(w, out, cout, 0, 0);
@@ -731,18 +876,22 @@ int mplbws_conv3x3_wgrad(const float* in, const float* dout, float* dw, float* d
         return MPLBWS_ERR_ARG;
     const int rows = wgrad_rows(h, wd);
     const int64_t chunks = (int64_t)n * ((h + rows - 1) / rows);
-    if (chunks > 65535) return MPLBWS_ERR_ARG;
+    // (a chunk's rows are addressed by 32-bit offsets)
+    if (chunks > 65535 || (int64_t)(rows + 2) * wd * std::max(cin, cout) >= (int64_t)1 << 30)
+        return MPLBWS_ERR_ARG;
     const int K = 9 * cin;
-    const dim3 grd((unsigned)((K + 31) / 32), (unsigned)((cout + 31) / 32), (unsigned)chunks);
     const int64_t cnt = (int64_t)K * cout;
     float* bp = dbias ? workspace + chunks * cnt : nullptr;
-    hipLaunchKernelGGL(k_conv_wgrad, grd, dim3(64 * kWaves), 0, 0, in, dout, workspace, bp, h,
-                       wd, cin, cout, rows);
-    hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)((cnt + 63) / 64)), dim3(64 * kSumWaves), 0,
-                       0, workspace, dw, cnt, (int)chunks);
-    if (dbias)
-        hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)((cout + 63) / 64)),
-                           dim3(64 * kSumWaves), 0, 0, bp, dbias, (int64_t)cout, (int)chunks);
+    const dim3 grd((unsigned)((cin + 31) / 32), (unsigned)((cout + 31) / 32), (unsigned)chunks);
+    if (vec4(in, dout, cin, cout, 0))
+        hipLaunchKernelGGL(k_conv_wgrad<true>, grd, dim3(64 * kGWaves), 0, 0, in, dout, workspace, bp,
+                           h, wd, cin, cout, rows);
+    else
+        hipLaunchKernelGGL(k_conv_wgrad<false>, grd, dim3(64 * kGWaves), 0, 0, in, dout, workspace,
+                           bp, h, wd, cin, cout, rows);
+    const int64_t sums = (cnt + 63) / 64 + (dbias ? (cout + 63) / 64 : 0);
+    hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)sums), dim3(64 * kSumWaves), 0, 0, workspace,
+                       dw, cnt, bp, dbias, (int64_t)cout, (int)chunks);
     return status();
 }
 

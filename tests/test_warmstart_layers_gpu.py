@@ -80,3 +80,31 @@ def test_convolution_forward(n, h, wd, cin, cout):
         # roundings of partial sums bounded by the sum of magnitudes
         tol = (9 * cin + 1) * 2.0 ** -24 * mag
         assert (np.abs(out.numpy() - ref) <= tol).all()
+
+
+# sub-tiles of 16 to 64 columns and their remainders, several segments of a
+# row, several chunks of an image (64 x 100 rows of 41), channels of one, two
+# and three tiles of 32 with remainders that are no multiple of 4
+@pytest.mark.parametrize("n,h,wd,cin,cout",
+                         [(1, 1, 1, 8, 4), (3, 2, 17, 5, 3), (2, 16, 16, 32, 32),
+                          (1, 33, 48, 40, 36), (2, 21, 65, 72, 24), (1, 9, 130, 8, 67),
+                          (2, 100, 64, 33, 12)])
+def test_convolution_weight_gradient(n, h, wd, cin, cout):
+    log("wgrad %s" % ((n, h, wd, cin, cout),))
+    lib, rng = ws.load(), np.random.default_rng(9)
+    A = ws.DeviceArray.from_numpy
+    x = rng.standard_normal((n, h, wd, cin)).astype(np.float32)
+    d = rng.standard_normal((n, h, wd, cout)).astype(np.float32)
+    dw, db = ws.DeviceArray((9, cin, cout)), ws.DeviceArray((cout,))
+    k = ws.DeviceArray((int(lib.mplbws_wgrad_workspace(n, h, wd, cin, cout)),))
+    ax, ad = A(x), A(d)
+    ck(lib.mplbws_conv3x3_wgrad(ax.p, ad.p, dw.p, db.p, k.p, n, h, wd, cin, cout))
+    ref, refb = nno.conv3x3_wgrad(x, d)
+    mag, magb = nno.conv3x3_wgrad(np.abs(x), np.abs(d))
+    # FP32 sums over the pixels, as for the forward convolution
+    m = n * h * wd
+    assert (np.abs(dw.numpy() - ref) <= m * 2.0 ** -24 * mag).all()
+    assert (np.abs(db.numpy() - refb) <= m * 2.0 ** -24 * magb + 1e-30).all()
+    again = ws.DeviceArray((9, cin, cout))
+    ck(lib.mplbws_conv3x3_wgrad(ax.p, ad.p, again.p, None, k.p, n, h, wd, cin, cout))
+    assert np.array_equal(again.numpy(), dw.numpy())
