@@ -61,13 +61,17 @@ __device__ __forceinline__ void march_wall(const MPLB_CONST RegionProg* progs,
 // 56 us at 5.4 TB/s); a march of K steps moves (64 / (64 - 2K)) (1 + 2K / rows)
 // reads and one write of the lattice per K steps.  One wave per workgroup and
 // no LDS, so no wave waits for another; K as many rows as the registers of W
-// waves per SIMD hold without a spill (FP64 K = 5 at W = 3, 8 at W = 2 was
-// 1.2 times slower).  Loads of the next row are issued before this row's
+// waves per SIMD hold and the ends of a strip leave worth it (2048^2, us per
+// step: FP32 K = 5 at W = 5 24.6, 6 at 4 26.4, 7 at 4 24.8, 8 at 4 27.8, 256
+// blocks of 104^2 20.3, 21.2, 19.4, 21.9; FP64 4 at 3 50.9, 5 at 3 46.7, 6 at 2
+// 50.3, 8 at 2 55.5; FP16 4 at 5 22.8, 5 at 4 23.3; with obstacles, 96 blocks
+// of 128^2, FP32 3 at 5 16.6, 4 at 4 15.7, 5 at 4 15.8, FP64 3 at 3 29.2, 4 at
+// 2 31.4).  Loads of the next row are issued before this row's
 // arithmetic; the wall constants come by scalar loads, and the rows that make
 // no result store out of range, since a vector load or a store under a branch
 // would make the wait for the row wait for those too.  us per step, single
-// steps and march (rows 16): FP32 2048^2 56 and 25.0 (K = 6), 256 blocks of
-// 128^2 92 and 39.4; FP64 2048^2 112 and 46 (K = 5); FP16 2048^2 34 and 22.8
+// steps and march (rows 16): FP32 2048^2 56 and 24.8 (K = 7), 256 blocks of 80
+// to 128 rows 92 and 39 (K = 6); FP64 2048^2 112 and 46 (K = 5); FP16 2048^2 34 and 22.8
 // (K = 4); FP32 with obstacles, 96 blocks of 128^2, 25.3 and 16.0 (K = 4).
 template <int ST, int K, bool OBST, int W>
 __global__ __launch_bounds__(64, W) void k_march(KParams kp) {
@@ -218,9 +222,9 @@ __global__ __launch_bounds__(64, W) void k_march(KParams kp) {
 // the forms: storage, obstacles, steps per launch, waves per SIMD
 #define MPLB_MARCH_FORMS(X)           \
     X(MPLBHIP_STORE_F64, false, 5, 3) \
-    X(MPLBHIP_STORE_F32, false, 6, 4) \
+    X(MPLBHIP_STORE_F32, false, 7, 4) \
     X(MPLBHIP_STORE_F16, false, 4, 5) \
-    X(MPLBHIP_STORE_F64, true, 4, 2)  \
+    X(MPLBHIP_STORE_F64, true, 3, 3)  \
     X(MPLBHIP_STORE_F32, true, 4, 4)  \
     X(MPLBHIP_STORE_F16, true, 4, 4)
 
