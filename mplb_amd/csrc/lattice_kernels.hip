@@ -823,23 +823,33 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce_blocks(
         double t = 0.0;
         for (int k = 0; k < kWaves; k++) t += red[k][threadIdx.x];
         out[(int64_t)b * kNAcc + threadIdx.x] = t;
+        if (nblocks == 1) out[kNAcc + threadIdx.x] = t;  // the total
     }
 }
 
-// the total over the blocks, in the same fixed-order fashion
+// the total over several blocks, in the same fixed-order fashion: the sums of
+// all kNAcc terms side by side, so the tree takes 8 barriers (term by
+// term it took 81 and 8.5 us); a single block needs no launch for it
 __global__ __launch_bounds__(256) void k_reduce_total(double* __restrict__ out, int nblocks) {
-    __shared__ double red[256];
-    for (int a = 0; a < kNAcc; a++) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += 256) s += out[(int64_t)b * kNAcc + a];
-        red[threadIdx.x] = s;
+    __shared__ double red[256][kNAcc];
+    double s[kNAcc];
+#pragma unroll
+    for (int a = 0; a < kNAcc; a++) s[a] = 0.0;
+    for (int b = threadIdx.x; b < nblocks; b += 256)
+#pragma unroll
+        for (int a = 0; a < kNAcc; a++) s[a] += out[(int64_t)b * kNAcc + a];
+#pragma unroll
+    for (int a = 0; a < kNAcc; a++) red[threadIdx.x][a] = s[a];
+    for (int o = 128; o > 0; o >>= 1) {
         __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
+        if ((int)threadIdx.x < o) {
+#pragma unroll
+            for (int a = 0; a < kNAcc; a++) red[threadIdx.x][a] += red[threadIdx.x + o][a];
         }
-        if (threadIdx.x == 0) out[(int64_t)nblocks * kNAcc + a] = red[0];
-        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int a = 0; a < kNAcc; a++) out[(int64_t)nblocks * kNAcc + a] = red[0][a];
     }
 }
 
@@ -988,7 +998,7 @@ hipError_t launch_reduce(const double* partials, const BlockParams* blocks, int 
                          hipStream_t s) {
     hipLaunchKernelGGL(k_reduce_blocks, dim3(nblocks), dim3(kRedThreads), 0, s, partials, blocks,
                        nblocks, ntiles, nbulk, nbnd, split, fold, out);
-    hipLaunchKernelGGL(k_reduce_total, dim3(1), dim3(256), 0, s, out, nblocks);
+    if (nblocks > 1) hipLaunchKernelGGL(k_reduce_total, dim3(1), dim3(256), 0, s, out, nblocks);
     return hipGetLastError();
 }
 
