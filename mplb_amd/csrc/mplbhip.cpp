@@ -1625,16 +1625,16 @@ static int assign_march(mplbhip_ctx* c, bool only_active) {
 //   FP32  512: 14.0, 3.9, 6.0    860: -, 8.3, 8.5        1024: 17.3, 10.6, 10.1
 // so tiles up to 2^20 nodes in FP64 and below that in reduced storage, where
 // k_march reads less per node, and above it where k_march cannot run
-// (2048 x 1024 periodic channel, single against tiles: FP64 57.4 and 43.2,
-// FP32 34.0 and 18.9).  The tile's side by the number of workgroups: small
-// ones while the chip has a CU for each (128^2 FP64: 1.7 with side 8, 2.2
-// with 16; 192^2: 3.1 and 2.5), the large, four-step ones when there are
-// several rounds of them (400^2 FP32: 3.1 either way; 512^2 FP64: 6.7 with
-// 16, 6.3 with 24).
+// (periodic or with a body force; 4096 x 2048 channel, single against tiles:
+// FP64 232 and 165, FP32 112 and 62, FP16 66 and 56).  The tile's side by the
+// number of workgroups: small ones while the chip has a CU for each (128^2
+// FP64: 1.7 with side 8, 2.2 with 16; 192^2: 3.1 and 2.5), the large,
+// four-step ones when there are several rounds of them (400^2 FP32: 3.1
+// either way; 512^2 FP64: 6.7 with 16, 6.3 with 24).
 static int assign_2d(mplbhip_ctx* c, bool only_active) {
     const int64_t most = c->storage == MPLBHIP_STORE_F64 ? 1 << 20 : (1 << 20) - 1;
     c->tile = c->tile_ok && c->pair_env >= 0 && c->pair_env != 2 &&
-              (c->grid_nodes <= most || !c->march_ok);
+              (c->grid_nodes <= most || !c->march_ok || c->force_type || c->force_macros);
     c->march = c->march_ok && c->pair_env >= 0 && !c->tile;
     return c->tile ? assign_tiles2d(c, only_active) : c->march ? assign_march(c, only_active) : 0;
 }

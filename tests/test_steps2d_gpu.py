@@ -119,6 +119,26 @@ def test_steps2d_channel_f64(size, monkeypatch):
     same_as_oracle(lambda be: cases.channel2d(be, size[0], size[1], 0.8, 1e-5), RUNS + (1, 17))
 
 
+@pytest.mark.parametrize("size", [(7, 30), (61, 44), (1040, 1020)])
+def test_steps2d_forced_cavity_f64(size, monkeypatch):
+    """A body force between four walls: tiles at every size."""
+    log("steps2d forced cavity %s" % (size,))
+
+    def build(be):
+        be.add_block(0, size)
+        be.set_collision(cases.tau_ref_for(0.8, 1.0), force_type=1, force_macros=True)
+        for s in ("Left", "Right", "Top", "Bottom"):
+            be.add_boundary(0, BS[s], BSch.EQMDiffuseRefl, (0.0, 0.01), VT.Wall)
+        be.prepare()
+        be.set_accel(0, (1e-5, -2e-5))
+        shp = tuple(reversed(size))
+        be.set_macros(0, cases.density_noise(shp), np.zeros(shp), np.zeros(shp))
+        be.init_feq()
+        be.set_dt(1.0)
+
+    same_as_oracle(build, RUNS if size[0] < 1000 else (6,))
+
+
 @pytest.mark.parametrize("storage", [hip.STORE_F32, hip.STORE_F16])
 def test_steps2d_channel_reduced_storage(storage, monkeypatch):
     same_as_single_steps(lambda be: cases.channel2d(be, 101, 60, 0.8, 1e-5), storage, "1",
