@@ -220,7 +220,7 @@ struct KParams {
     // the swap scheme: the buffer written (0 but within a run of k_swap_pull),
     // and the masks of every block's regions
     int32_t swap_to;
-    const uint2* swap_mask;
+    const uint32_t* swap_mask;  // two words per region
 };
 
 struct HaloParams {

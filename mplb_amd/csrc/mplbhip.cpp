@@ -353,7 +353,7 @@ static KParams base_params(mplbhip_ctx* c) {
     kp.ntile2d = c->ntile2d;
     kp.tile_row = c->tile_row;
     kp.wrap_x = c->wrap_x ? 1 : 0;
-    kp.swap_mask = static_cast<const uint2*>(c->swap_mask.p);
+    kp.swap_mask = static_cast<const uint32_t*>(c->swap_mask.p);
     return kp;
 }
 

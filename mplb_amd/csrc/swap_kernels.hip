@@ -366,7 +366,8 @@ __global__ __launch_bounds__(kTX* kTY) void k_swap_pull(KParams kp, int nbnd) {
     double f[Q];
     if (bnd) {
         const int t = (int)threadIdx.y * kTX + (int)threadIdx.x;
-        if (t < 27) s_mask[t] = kp.swap_mask[r.b * 27 + t];
+        if (t < 54)
+            reinterpret_cast<uint32_t*>(s_mask)[t] = kp.swap_mask[r.b * 54 + t];
         __syncthreads();
         if (!r.active) return;
         const int rx = region_code(r.x, B.n[0]) + 3 * region_code(r.y, B.n[1]) +
