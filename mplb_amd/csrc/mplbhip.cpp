@@ -2257,9 +2257,14 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         return 0;
     }
     // untimed: replay captured graphs of G steps (even, so the parity after
-    // a graph is unchanged; MPLBHIP_GRAPH_STEPS overrides 32), the
-    // remainder one by one
-    int G = 32;
+    // a graph of single steps is unchanged; MPLBHIP_GRAPH_STEPS overrides),
+    // the remainder launch by launch.  32 steps, or 16 launches of several:
+    // replaying a graph costs some 10 us more than its launches one by one,
+    // which a run of fewer than 16 takes as fast (2D cavity 128^2, FP64, 100
+    // steps between checks: 1,000 steps in 2.18 ms with graphs of 4 launches,
+    // 2.09 of 8, 2.11 of 16, that is none).
+    const int ls = launch_steps(c);
+    int G = std::max(32, 16 * ls);
     if (const char* e = std::getenv("MPLBHIP_GRAPH_STEPS")) {
         const int g = std::atoi(e);
         if (g >= 2 && g <= 1024 && g % 2 == 0) G = g;
@@ -2271,7 +2276,7 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         left--;
     }
     // launches of several steps leave the last step to a single one
-    const int ls = launch_steps(c), keep = ls > 1 && !tail ? 1 : 0;
+    const int keep = ls > 1 && !tail ? 1 : 0;
     G -= G % ls;  // whole launches
     if (G > 0 && left - keep >= G) {
         if (c->graph_steps != G)

@@ -22,7 +22,7 @@ TILE = [(3, 3), (8, 17), (16, 40), (33, 8), (120, 130), (150, 131)]
 # one to four row groups per wave, a strip and its edges, several strips
 MARCH = [(3, 3), (5, 70), (17, 33), (33, 40), (64, 9), (65, 16), (131, 17), (600, 31)]
 FORMS = [("1", s) for s in TILE] + [("2", s) for s in MARCH]
-RUNS = (1, 2, 3, 9, 40)  # alone, in one short launch, a graph replay and a rest
+RUNS = (1, 2, 3, 9, 40)  # alone, in one short launch, in several and a rest
 
 
 def log(m):
@@ -153,6 +153,16 @@ def test_steps2d_obstacles(n, form, storage, monkeypatch):
     rects = [(4, 5, 6, 3), (n // 2, n // 3, 5, 7)]
     same_as_single_steps(lambda be: cases.cavity2d_obstacles(be, n, rects), storage, form,
                          monkeypatch)
+
+
+@pytest.mark.parametrize("form", ["1", "2"])
+def test_steps2d_graph_replays_f64(form, monkeypatch):
+    """Runs of whole graphs of 16 launches, with and without a rest, and the
+    single steps after them; the periodic channel's halos too."""
+    monkeypatch.setenv("MPLBHIP_PAIR", form)
+    same_as_oracle(lambda be: cavity(be, (70, 19)), (300, 129, 1, 131))
+    if form == "1":
+        same_as_oracle(lambda be: cases.channel2d(be, 45, 18, 0.8, 1e-5), (257, 2, 140))
 
 
 @pytest.mark.parametrize("form", ["1", "2"])
