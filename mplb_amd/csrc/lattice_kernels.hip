@@ -1011,6 +1011,24 @@ __global__ __launch_bounds__(256) void k_copy16(const u32x4* __restrict__ src,
         __builtin_nontemporal_store(src[i], dst + i);
 }
 
+// exchange the contents of two buffers
+__global__ void k_exchange(uint32_t* a, uint32_t* b, int64_t n) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t v = a[i];
+        a[i] = b[i];
+        b[i] = v;
+    }
+}
+
+hipError_t launch_exchange(void* a, void* b, int64_t bytes, hipStream_t s) {
+    const int64_t n = bytes / 4;
+    const int64_t grid = std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 65536));
+    hipLaunchKernelGGL(k_exchange, dim3((unsigned)grid), dim3(256), 0, s,
+                       static_cast<uint32_t*>(a), static_cast<uint32_t*>(b), n);
+    return hipGetLastError();
+}
+
 hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t s) {
     // one 16-byte element per thread up to 16 GiB (a grid-stride loop
     // over 8192 workgroups copied 2 GiB at 4.75 TB/s, this form at 6.28)

@@ -40,6 +40,7 @@ hipError_t launch_fill(void* p, int64_t bytes, hipStream_t s);
 hipError_t launch_lift(int dim, const KParams& kp, int64_t nodes, hipStream_t s);
 hipError_t launch_rest_macros(const KParams& kp, int b, int64_t nodes, hipStream_t s);
 hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t s);
+hipError_t launch_exchange(void* a, void* b, int64_t bytes, hipStream_t s);
 hipError_t scratch_address(double** ptr);
 bool swap_masks(const RegionProg* progs, uint32_t* mask);
 hipError_t launch_swap_pull(const KParams& kp, int nbnd, bool collide, bool large, hipStream_t s);
@@ -102,6 +103,7 @@ struct mplbhip_ctx {
 
     // layout
     std::vector<BlockParams> bp;
+    std::vector<int64_t> elem0;  // first element of each block's storage, and the end
     int64_t total_elems = 0;
     int64_t interior_nodes = 0;
     int ntiles = 0;            // whole-lattice tiles
@@ -1720,6 +1722,7 @@ int mplbhip_prepare(mplbhip_ctx* c) {
     const int hz = c->dim == 3 ? 1 : 0;
     const int align = (int)(128 / c->es);
     c->bp.assign(nb, BlockParams{});
+    c->elem0.assign(1, 0);
     int64_t off = 0, moff = 0;
     c->segs.clear();
     // measured at 256^3: folding the x faces pays for 4- and 8-byte
@@ -1760,6 +1763,7 @@ int mplbhip_prepare(mplbhip_ctx* c) {
         B.sq = (int32_t)sq;
         B.base = off + hz * sz + sx + ox;
         off += (elems + 255) / 256 * 256;
+        c->elem0.push_back(off);
         {
             const int (*cv)[3] = lattice_tab(c->lat).C;
             const int64_t shift = (c->dim == 3 ? sz : 0) + sx + 1;
@@ -2428,6 +2432,39 @@ static int restart_at_rest(mplbhip_ctx* c, const std::vector<int>& blocks) {
     return 0;
 }
 
+// Bring every block to the buffer c->cur.  A frozen instance keeps its parity
+// while the launches go on, and the halo copies take one buffer for every
+// block (exchange), so an instance that stopped an odd number of launches
+// before the others has its two buffers exchanged, whole: halos, the step
+// before the latest, kept boundary populations.
+static int align_parity(mplbhip_ctx* c) {
+    const size_t nb = c->bp.size();
+    std::vector<int32_t> par(nb);
+    HIPCHK(c, hipMemcpyAsync(par.data(), c->parity[c->cur].p, nb * sizeof(int32_t),
+                             hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const size_t slot = c->Q * (c->storage == MPLBHIP_STORE_F64 ? 8 : 4);
+    auto exchange = [&](DevBuf* pair, size_t at, size_t bytes) {
+        return launch_exchange(static_cast<char*>(pair[0].p) + at,
+                               static_cast<char*>(pair[1].p) + at, (int64_t)bytes, c->stream);
+    };
+    for (size_t b = 0; b < nb; b++) {
+        if (par[b] == c->cur) continue;
+        HIPCHK(c, exchange(c->fs, c->elem0[b] * c->es, (c->elem0[b + 1] - c->elem0[b]) * c->es));
+        for (int r = 1; r < c->plan.nregions; r++) {
+            const size_t i = b * c->plan.nregions + r;
+            if (c->plan.progs[i].persist >= 0)
+                HIPCHK(c, exchange(c->per, c->plan.progs[i].persist * slot,
+                                   c->plan.persist_nodes[i] * slot));
+        }
+        par[b] = c->cur;
+    }
+    HIPCHK(c, hipMemcpyAsync(c->parity[c->cur].p, par.data(), nb * sizeof(int32_t),
+                             hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+}
+
 int mplbhip_iterate_batch(mplbhip_ctx* c, double criteria, int check_period,
                           long long max_steps, long long* steps_b, double* res_b,
                           long long* steps_done) {
@@ -2575,6 +2612,8 @@ int mplbhip_iterate_batch(mplbhip_ctx* c, double criteria, int check_period,
     if (frozen)
         HIPCHK(c, hipMemcpyAsync(c->blocks.p, c->bp.data(), nb * sizeof(BlockParams),
                                  hipMemcpyHostToDevice, c->stream));
+    if (frozen && !c->halos.empty())
+        if (int rc = align_parity(c)) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (steps_b)
         for (int b = 0; b < nb; b++) steps_b[b] = conv[b];
