@@ -646,81 +646,63 @@ __global__ void k_pool_bwd(const float* __restrict__ dout, float* __restrict__ d
     }
 }
 
-// Where these two and k_channels had an element per iteration with the 64-bit
-// divisions of its whole index (some 100 instructions each), a workgroup now
-// takes one coarse row or 64 pixels and an item's place in it is one 32-bit
-// division; HBM bounds them.
+// These three take their items (V channels of a pixel) by one 32-bit index over
+// all of them, with 32-bit divisions (some 20 instructions each; of 64-bit
+// ones, 100); the host cuts larger calls into slabs (slabs).  HBM bounds them.
+constexpr int64_t kSlab = (int64_t)1 << 30;
 
-// nearest 2x upsampling (h, wd: the coarse size) into channels [c0, c0+c)
-// of a tensor with ctot channels, and its adjoint: one coarse row per
-// workgroup and iteration, every coarse value read once.  32 images of 64 x 64
-// x 48 to 128 x 128 x 72: 79.7 -> 20.9 us (6.0 TB/s).
+// nearest 2x upsampling (wd: the coarse width) of items / (cols cv) rows of
+// cols columns into channels of a tensor with ctot channels, and its adjoint.
+// (fine row 2 y of image b is row 2 (b h + y) of all)
+// 32 images of 64 x 64 x 48 and 128 x 128 x 72, forward 18.5 us (one channel
+// and an index of 64 bits: 73), backward 23.5 (four channels: 25.1).
 template <int V>
-__global__ void k_up_fwd(const float* __restrict__ in, float* __restrict__ out, int64_t rows,
-                         int wd, int c, int ctot, int c0) {
-    const uint32_t cv = (uint32_t)c / V, items = (uint32_t)wd * cv;
-    const int64_t W = 2 * (int64_t)wd;
-    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
-        // (fine row 2 y of image b is row 2 (b h + y) of all)
-        float* fine = out + 2 * r * W * ctot + c0;
-        const float* coarse = in + r * wd * c;
-        for (uint32_t i = threadIdx.x; i < items; i += blockDim.x) {
-            const uint32_t x = i / cv, k = (i - x * cv) * V;
-            const Vec<V> v = Vec<V>::ld(coarse + (int64_t)i * V);
-            float* f = fine + 2 * (int64_t)x * ctot + k;
-            v.st(f);
-            v.st(f + ctot);
-            v.st(f + W * ctot);
-            v.st(f + W * ctot + ctot);
-        }
+__global__ void k_up_fwd(const float* __restrict__ in, float* __restrict__ out, uint32_t items,
+                         uint32_t cols, uint32_t cv, int wd, int ctot) {
+    const int64_t W = 2 * (int64_t)wd, c = (int64_t)cv * V;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < items; i += gridDim.x * 256u) {
+        const uint32_t q = i / cv, k = (i - q * cv) * V, r = q / cols, x = q - r * cols;
+        const Vec<V> v = Vec<V>::ld(in + ((int64_t)r * wd + x) * c + k);
+        float* f = out + (2 * (int64_t)r * W + 2 * (int64_t)x) * ctot + k;
+        v.st(f);
+        v.st(f + ctot);
+        v.st(f + W * ctot);
+        v.st(f + W * ctot + ctot);
     }
 }
 
-template <int V>
-__global__ void k_up_bwd(const float* __restrict__ dout, float* __restrict__ din, int64_t rows,
-                         int wd, int c, int ctot, int c0) {
-    const uint32_t cv = (uint32_t)c / V, items = (uint32_t)wd * cv;
+__global__ void k_up_bwd(const float* __restrict__ dout, float* __restrict__ din, uint32_t items,
+                         uint32_t cols, uint32_t c, int wd, int ctot) {
     const int64_t W = 2 * (int64_t)wd;
-    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
-        const float* fine = dout + 2 * r * W * ctot + c0;
-        float* coarse = din + r * wd * c;
-        for (uint32_t i = threadIdx.x; i < items; i += blockDim.x) {
-            const uint32_t x = i / cv, k = (i - x * cv) * V;
-            const float* f = fine + 2 * (int64_t)x * ctot + k;
-            const Vec<V> a = Vec<V>::ld(f), b = Vec<V>::ld(f + ctot);
-            const Vec<V> d = Vec<V>::ld(f + W * ctot), e = Vec<V>::ld(f + W * ctot + ctot);
-            Vec<V> o;
-#pragma unroll
-            for (int j = 0; j < V; j++) o.v[j] = (a.v[j] + b.v[j]) + (d.v[j] + e.v[j]);
-            o.st(coarse + (int64_t)i * V);
-        }
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < items; i += gridDim.x * 256u) {
+        const uint32_t q = i / c, k = i - q * c, r = q / cols, x = q - r * cols;
+        const float* f = dout + (2 * (int64_t)r * W + 2 * (int64_t)x) * ctot + k;
+        din[((int64_t)r * wd + x) * c + k] =
+            (f[0] + f[ctot]) + (f[W * ctot] + f[W * ctot + ctot]);
     }
 }
 
 // copy channels [0, c) of src (c channels) into channels [c0, c0 + c) of
 // dst (ctot channels) (dir = 0), or back (dir = 1), or add them back (dir =
-// 2): 64 pixels per workgroup and iteration.  32 images of 128 x 128 x 24
-// into 72: 19.7 -> 17.3 us (5.8 TB/s).
+// 2); the tensor of ctot channels from channel c0 on.  32 images of 128 x 128
+// x 24 into 72: 15.6 us (one channel and an index of 64 bits: 18.6).
 template <int V>
-__global__ void k_channels(const float* __restrict__ a, float* __restrict__ b, int64_t pixels,
-                           int c, int ctot, int c0, int dir) {
-    const uint32_t cv = (uint32_t)c / V;
-    for (int64_t p0 = (int64_t)blockIdx.x * 64; p0 < pixels; p0 += (int64_t)gridDim.x * 64) {
-        const uint32_t items = (uint32_t)(pixels - p0 < 64 ? pixels - p0 : 64) * cv;
-        for (uint32_t i = threadIdx.x; i < items; i += blockDim.x) {
-            const uint32_t p = i / cv, k = (i - p * cv) * V;
-            const int64_t thin = (p0 + p) * c + k, wide = (p0 + p) * ctot + c0 + k;
-            if (dir == 0) {
-                Vec<V>::ld(a + thin).st(b + wide);
-            } else {
-                Vec<V> v = Vec<V>::ld(a + wide);
-                if (dir != 1) {
-                    const Vec<V> o = Vec<V>::ld(b + thin);
+__global__ void k_channels(const float* __restrict__ a, float* __restrict__ b, uint32_t items,
+                           uint32_t cv, int ctot, int dir) {
+    const int64_t c = (int64_t)cv * V;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < items; i += gridDim.x * 256u) {
+        const uint32_t p = i / cv, k = (i - p * cv) * V;
+        const int64_t thin = p * c + k, wide = (int64_t)p * ctot + k;
+        if (dir == 0) {
+            Vec<V>::ld(a + thin).st(b + wide);
+        } else {
+            Vec<V> v = Vec<V>::ld(a + wide);
+            if (dir != 1) {
+                const Vec<V> o = Vec<V>::ld(b + thin);
 #pragma unroll
-                    for (int j = 0; j < V; j++) v.v[j] = o.v[j] + v.v[j];
-                }
-                v.st(b + thin);
+                for (int j = 0; j < V; j++) v.v[j] = o.v[j] + v.v[j];
             }
+            v.st(b + thin);
         }
     }
 }
@@ -813,6 +795,20 @@ int grid_for(int64_t total) {
 bool vec4(const void* p, const void* q, int64_t c, int64_t ctot, int64_t c0) {
     return ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(q)) & 15) == 0 &&
            ((c | ctot | c0) & 3) == 0;
+}
+
+// launch(first row, first column, items, columns, cv, grid) over rows of wd
+// columns of cv items, in slabs of at most kSlab items (or of one column)
+// (8192 workgroups that loop against one per 256 items: 32.5 and 42 us for
+// 32 images of 128 x 128 x 47 channels into 72, one at a time)
+template <typename F> void slabs(int64_t rows, int64_t wd, int64_t cv, const F& launch) {
+    const int64_t cols = std::max<int64_t>(1, std::min(wd, kSlab / cv));
+    const int64_t some = std::max<int64_t>(1, std::min(rows, kSlab / (cols * cv)));
+    for (int64_t r = 0; r < rows; r += some)
+        for (int64_t x = 0; x < wd; x += cols) {
+            const int64_t nc = std::min(cols, wd - x), items = std::min(some, rows - r) * nc * cv;
+            launch(r, x, (uint32_t)items, (uint32_t)nc, (uint32_t)cv, dim3(grid_for(items)));
+        }
 }
 
 int status() { return hipGetLastError() == hipSuccess ? 0 : MPLBWS_ERR_HIP; }
@@ -917,36 +913,42 @@ int mplbws_pool2_bwd(const float* dout, float* din, int n, int h, int wd, int c)
 
 int mplbws_up2_fwd(const float* in, float* out, int n, int h, int wd, int c, int ctot, int c0) {
     if (!in || !out || c0 < 0 || c0 + c > ctot) return MPLBWS_ERR_ARG;
-    const int64_t rows = (int64_t)n * h;
-    const dim3 grd((unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, 65536)));
-    if (vec4(in, out, c, ctot, c0))
-        hipLaunchKernelGGL(k_up_fwd<4>, grd, dim3(256), 0, 0, in, out, rows, wd, c, ctot, c0);
-    else
-        hipLaunchKernelGGL(k_up_fwd<1>, grd, dim3(256), 0, 0, in, out, rows, wd, c, ctot, c0);
+    if (n <= 0 || h <= 0 || wd <= 0 || c <= 0) return status();
+    const bool v4 = vec4(in, out, c, ctot, c0);
+    slabs((int64_t)n * h, wd, v4 ? c / 4 : c, [&](int64_t r, int64_t x, uint32_t items,
+                                                  uint32_t cols, uint32_t cv, dim3 grd) {
+        const float* i = in + (r * wd + x) * c;
+        float* o = out + (4 * r * wd + 2 * x) * ctot + c0;
+        if (v4) hipLaunchKernelGGL(k_up_fwd<4>, grd, dim3(256), 0, 0, i, o, items, cols, cv, wd, ctot);
+        else hipLaunchKernelGGL(k_up_fwd<1>, grd, dim3(256), 0, 0, i, o, items, cols, cv, wd, ctot);
+    });
     return status();
 }
 
 int mplbws_up2_bwd(const float* dout, float* din, int n, int h, int wd, int c, int ctot, int c0) {
     if (!dout || !din || c0 < 0 || c0 + c > ctot) return MPLBWS_ERR_ARG;
-    const int64_t rows = (int64_t)n * h;
-    const dim3 grd((unsigned)std::max<int64_t>(1, std::min<int64_t>(rows, 65536)));
-    if (vec4(dout, din, c, ctot, c0))
-        hipLaunchKernelGGL(k_up_bwd<4>, grd, dim3(256), 0, 0, dout, din, rows, wd, c, ctot, c0);
-    else
-        hipLaunchKernelGGL(k_up_bwd<1>, grd, dim3(256), 0, 0, dout, din, rows, wd, c, ctot, c0);
+    if (n <= 0 || h <= 0 || wd <= 0 || c <= 0) return status();
+    slabs((int64_t)n * h, wd, c, [&](int64_t r, int64_t x, uint32_t items, uint32_t cols, uint32_t,
+                                     dim3 grd) {
+        hipLaunchKernelGGL(k_up_bwd, grd, dim3(256), 0, 0, dout + (4 * r * wd + 2 * x) * ctot + c0,
+                           din + (r * wd + x) * c, items, cols, (uint32_t)c, wd, ctot);
+    });
     return status();
 }
 
 int mplbws_channels(const float* src, float* dst, int64_t pixels, int c, int ctot, int c0,
                     int direction) {
     if (!src || !dst || c0 < 0 || c0 + c > ctot) return MPLBWS_ERR_ARG;
-    const dim3 grd((unsigned)std::max<int64_t>(1, std::min<int64_t>((pixels + 63) / 64, 65536)));
-    if (vec4(src, dst, c, ctot, c0))
-        hipLaunchKernelGGL(k_channels<4>, grd, dim3(256), 0, 0, src, dst, pixels, c, ctot, c0,
-                           direction);
-    else
-        hipLaunchKernelGGL(k_channels<1>, grd, dim3(256), 0, 0, src, dst, pixels, c, ctot, c0,
-                           direction);
+    if (pixels <= 0 || c <= 0) return status();
+    const bool v4 = vec4(src, dst, c, ctot, c0);
+    slabs(pixels, 1, v4 ? c / 4 : c, [&](int64_t p, int64_t, uint32_t items, uint32_t, uint32_t cv,
+                                         dim3 grd) {
+        const int64_t thin = p * c, wide = p * ctot + c0;
+        const float* a = src + (direction == 0 ? thin : wide);
+        float* b = dst + (direction == 0 ? wide : thin);
+        if (v4) hipLaunchKernelGGL(k_channels<4>, grd, dim3(256), 0, 0, a, b, items, cv, ctot, direction);
+        else hipLaunchKernelGGL(k_channels<1>, grd, dim3(256), 0, 0, a, b, items, cv, ctot, direction);
+    });
     return status();
 }
 

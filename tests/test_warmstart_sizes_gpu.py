@@ -1,0 +1,99 @@
+"""The warm-start network's layers away from the square images of the network:
+sizes of nothing, images of few rows or columns, arrays past 32-bit offsets."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from mplb_amd import warmstart as ws
+from oracle import nn_oracle as nno
+
+pytestmark = pytest.mark.gpu
+
+
+def log(m):
+    print(m, flush=True)
+
+
+def ck(rc):
+    assert rc == 0, rc
+
+
+def at(d, offset):
+    """Element `offset` of a device array."""
+    return ctypes.c_void_p(d.p.value + 4 * offset)
+
+
+# no image, no row, no column, no channel; all that is none is negative too
+@pytest.mark.parametrize("n,h,wd,c", [(0, 2, 2, 4), (2, 0, 2, 4), (2, 2, 0, 4), (2, 2, 2, 0),
+                                      (-1, 2, 2, 4), (2, -2, 2, 4), (2, 2, -2, 4), (2, 2, 2, -4),
+                                      (2, 2, 2, -3)])
+def test_upsampling_and_channel_copies_of_nothing(n, h, wd, c):
+    log("nothing %s" % ((n, h, wd, c),))
+    lib, rng = ws.load(), np.random.default_rng(3)
+    a, b = (rng.standard_normal((2, 4, 4, 8)).astype(np.float32) for _ in range(2))
+    da, db = ws.DeviceArray.from_numpy(a), ws.DeviceArray.from_numpy(b)
+    ck(lib.mplbws_up2_fwd(da.p, db.p, n, h, wd, c, 8, 0))
+    ck(lib.mplbws_up2_bwd(da.p, db.p, n, h, wd, c, 8, 0))
+    for direction in range(3):
+        ck(lib.mplbws_channels(da.p, db.p, n * h * wd, c, 8, 0, direction)
+           if c <= 0 or n * h * wd <= 0 else 0)
+    assert np.array_equal(da.numpy(), a) and np.array_equal(db.numpy(), b)
+
+
+# one row, one column, more channels than pixels; an index past 2^30 items
+@pytest.mark.parametrize("rows,wd,c,ctot,c0", [(1, 3000, 16, 24, 8), (3000, 1, 5, 7, 1),
+                                               (1, 1, 20000, 20004, 4), (2, 3, 1031, 1031, 0)])
+def test_upsampling_and_channel_copies_of_thin_images(rows, wd, c, ctot, c0):
+    log("thin %s" % ((rows, wd, c, ctot, c0),))
+    lib, rng = ws.load(), np.random.default_rng(4)
+    A = ws.DeviceArray.from_numpy
+    x = rng.standard_normal((1, rows, wd, c)).astype(np.float32)
+    wide = rng.standard_normal((1, 2 * rows, 2 * wd, ctot)).astype(np.float32)
+    dx, dw = A(x), A(wide)
+    ck(lib.mplbws_up2_fwd(dx.p, dw.p, 1, rows, wd, c, ctot, c0))
+    ref = wide.copy()
+    ref[..., c0:c0 + c] = x.repeat(2, axis=1).repeat(2, axis=2)
+    assert np.array_equal(dw.numpy(), ref)
+    dw = A(wide)
+    ck(lib.mplbws_up2_bwd(dw.p, dx.p, 1, rows, wd, c, ctot, c0))
+    f = wide[..., c0:c0 + c]
+    assert np.array_equal(dx.numpy(), (f[:, ::2, ::2] + f[:, ::2, 1::2])
+                          + (f[:, 1::2, ::2] + f[:, 1::2, 1::2]))
+    thin = ws.DeviceArray((1, 2 * rows, 2 * wd, c))
+    ck(lib.mplbws_channels(dw.p, thin.p, 4 * rows * wd, c, ctot, c0, 1))
+    assert np.array_equal(thin.numpy(), f)
+
+
+def test_upsampling_and_channel_copies_past_two_to_the_thirty_items():
+    """One channel, so an item per pixel: the last pixels of 2^30 + 4096, in a
+    few long rows and in many short ones."""
+    lib, rng = ws.load(), np.random.default_rng(6)
+    total, tail = (1 << 30) + 4096, 256
+    v = rng.standard_normal(tail).astype(np.float32)
+    coarse, fine = ws.DeviceArray((total,)), ws.DeviceArray((4 * total,))
+
+    def put(d, offset, a):
+        ck(lib.mplbws_upload(at(d, offset), a.ctypes.data, a.nbytes))
+
+    def get(d, offset, count):
+        out = np.empty(count, np.float32)
+        ck(lib.mplbws_download(out.ctypes.data, at(d, offset), out.nbytes))
+        return out
+
+    for rows in (1, total // 4096):
+        log("up %d x %d" % (rows, total // rows))
+        wd = total // rows
+        put(coarse, total - tail, v)
+        ck(lib.mplbws_zero(fine.p, 4 * fine.numel()))
+        ck(lib.mplbws_up2_fwd(coarse.p, fine.p, 1, rows, wd, 1, 1, 0))
+        for row in (1, 2):  # the last two fine rows
+            end = 4 * total - (row - 1) * 2 * wd
+            assert np.array_equal(get(fine, end - 2 * tail, 2 * tail), v.repeat(2))
+        put(coarse, total - tail, np.zeros(tail, np.float32))
+        ck(lib.mplbws_up2_bwd(fine.p, coarse.p, 1, rows, wd, 1, 1, 0))
+        assert np.array_equal(get(coarse, total - tail, tail), 4 * v)
+    put(coarse, total - tail, np.zeros(tail, np.float32))
+    put(fine, total - tail, v)
+    ck(lib.mplbws_channels(fine.p, coarse.p, total, 1, 1, 0, 1))
+    assert np.array_equal(get(coarse, total - tail, tail), v)
