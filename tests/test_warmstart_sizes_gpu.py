@@ -97,3 +97,22 @@ def test_upsampling_and_channel_copies_past_two_to_the_thirty_items():
     put(fine, total - tail, v)
     ck(lib.mplbws_channels(fine.p, coarse.p, total, 1, 1, 0, 1))
     assert np.array_equal(get(coarse, total - tail, tail), v)
+
+
+# one to seven rows, in tiles of more than 32 columns: one column short of a
+# tile, a tile, several with a remainder, and enough images for larger tiles
+@pytest.mark.parametrize("n,h,wd,cin,cout", [(1, 1, 66, 8, 4), (2, 1, 67, 16, 8), (530, 1, 111, 8, 4),
+                                             (2, 2, 99, 8, 33), (1, 3, 39, 40, 8),
+                                             (300, 2, 166, 8, 8), (1, 5, 101, 8, 5),
+                                             (3, 7, 70, 24, 24)])
+def test_convolution_of_few_rows(n, h, wd, cin, cout):
+    log("conv %s" % ((n, h, wd, cin, cout),))
+    lib, rng = ws.load(), np.random.default_rng(11)
+    A = ws.DeviceArray.from_numpy
+    x = rng.standard_normal((n, h, wd, cin)).astype(np.float32)
+    w = (rng.standard_normal((9, cin, cout)) / 8).astype(np.float32)
+    dx, dw, out = A(x), A(w), ws.DeviceArray((n, h, wd, cout))
+    ck(lib.mplbws_conv3x3_fwd(dx.p, dw.p, None, out.p, n, h, wd, cin, cout, 0))
+    # FP32 sums of 9 cin exact products
+    tol = (9 * cin + 1) * 2.0 ** -24 * nno.conv3x3(np.abs(x), np.abs(w))
+    assert (np.abs(out.numpy() - nno.conv3x3(x, w)) <= tol).all()
