@@ -337,13 +337,14 @@ __host__ __device__ inline int wgrad_rows(int h, int wd) {
 // Weight gradient partials of one chunk of whole rows: partial[chunk][tap][ci]
 // [co] = sum over its pixels m of in[shift_tap(m)][ci] dout[m][co], products
 // of 16 pixels.  A workgroup takes 32 input and 32 output channels, one wave
-// per tap; sub-tiles of at most kGPix pixels (RT rows of SEG columns, a
+// per tap; sub-tiles of at most kGPix pixels (RT lines of SEG positions, a
 // multiple of 16) of dout, and of the input with a pixel around them, are
 // converted to BF16 once into LDS as they lie in HBM, a pixel's 32 channels in
 // a row, and read transposed (ds_read_b64_tr_b16): the product's reduction
 // runs over pixels, and a tap is a shift by whole pixels, which needs no
-// alignment.  The workgroups of the first input channels also sum the dout
-// values they load (FP32, fixed order) into bpart[chunk][co] when it is given.
+// alignment.  Lines are the chunk's rows, or (TURN) its columns.  The
+// workgroups of the first input channels also sum the dout values they load
+// (FP32, fixed order) into bpart[chunk][co] when it is given.
 //
 // Bound: the loads of one sub-tile per workgroup in flight, and too few
 // workgroups for the chip when the chunks are few (one image of 64 x 64: 2 us
@@ -355,18 +356,24 @@ __host__ __device__ inline int wgrad_rows(int h, int wd) {
 // tiles summed in LDS took 52 to 103, its staging three times as much.
 constexpr int kGWaves = 9;
 constexpr int kGPix = 256;   // pixels of dout staged
-constexpr int kGIn = 396;    // and of the input: (RT + 2)(SEG + 2), 4 rows of 64 the most
+constexpr int kGIn = 396;    // and of the input: (RT + 2)(SEG + 2), 4 lines of 64 the most
 
-// columns and rows of a sub-tile
+// positions and lines of a sub-tile
 struct GradTile {
     int seg, segs, rt;
 };
-__host__ __device__ inline GradTile grad_tile(int wd) {
+__host__ __device__ inline GradTile grad_tile(int lines, int positions) {
     GradTile t;
-    t.segs = (wd + 63) / 64;
-    t.seg = ((wd + t.segs - 1) / t.segs + 15) / 16 * 16;
-    t.rt = kGPix / t.seg;
+    const int most = lines == 1 ? 128 : lines == 2 ? 96 : 64;
+    t.segs = (positions + most - 1) / most;
+    t.seg = ((positions + t.segs - 1) / t.segs + 15) / 16 * 16;
+    t.rt = kGPix / t.seg < lines ? kGPix / t.seg : lines;
     return t;
+}
+// sub-tiles of a chunk
+inline int64_t grad_tiles(int lines, int positions) {
+    const GradTile t = grad_tile(lines, positions);
+    return (int64_t)((lines + t.rt - 1) / t.rt) * t.segs;
 }
 
 // four pixels of one channel: the 16 lanes of a row each point at 4 channels
@@ -376,25 +383,30 @@ __device__ __forceinline__ s16x4 lds_tr(const short* p) {
 }
 
 // 8 channels at a byte offset, `left` of them (a multiple of 4 if VEC) real;
-// zeros past them and for off = bytes
+// zeros past them and for off = bytes.  Without VEC the loads are as wide, at
+// any multiple of four bytes, and what is not this pixel's is dropped (8
+// images of 64 x 64, 35 to 33 channels: 105 us by single floats, 48).
 template <bool VEC>
 __device__ __forceinline__ void load8(float4* f, __amdgpu_buffer_rsrc_t r, uint32_t off, int left,
                                       uint32_t bytes) {
-    if constexpr (VEC) {
-        f[0] = buf_ld4(r, left > 0 ? off : bytes, 0);
-        f[1] = buf_ld4(r, left > 4 ? off + 16u : bytes, 0);
-    } else {
-        float v[8];
-#pragma unroll
-        for (int c = 0; c < 8; c++) v[c] = buf_ld1(r, left > c ? off + 4u * c : bytes, 0);
-        f[0] = float4{v[0], v[1], v[2], v[3]};
-        f[1] = float4{v[4], v[5], v[6], v[7]};
+    f[0] = buf_ld4(r, left > 0 ? off : bytes, 0);
+    f[1] = buf_ld4(r, left > 4 ? off + 16u : bytes, 0);
+    if constexpr (!VEC) {
+        f[0].y = left > 1 ? f[0].y : 0.f;
+        f[0].z = left > 2 ? f[0].z : 0.f;
+        f[0].w = left > 3 ? f[0].w : 0.f;
+        f[1].y = left > 5 ? f[1].y : 0.f;
+        f[1].z = left > 6 ? f[1].z : 0.f;
+        f[1].w = left > 7 ? f[1].w : 0.f;
     }
 }
 
 // VEC: cin and cout are multiples of four, in and dout aligned for 16-byte
-// accesses
-template <bool VEC>
+// accesses.
+// TURN: where the chunk is in fewer sub-tiles by columns than by rows (1 x 4096
+// pixels by rows would be 256 sub-tiles of 16 columns each, one of them real:
+// 64 to 64 channels 1270 us, 55; 8 columns 166, 40).
+template <bool VEC, bool TURN>
 __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __restrict__ in,
                                                                 const float* __restrict__ dout,
                                                                 float* __restrict__ partial,
@@ -405,26 +417,32 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
     // [pixel][32 channels]
     __shared__ __attribute__((aligned(16))) short s_x[kGIn * 32];
     __shared__ __attribute__((aligned(16))) short s_d[kGPix * 32];
-    const GradTile T = grad_tile(wd);
     const int lane = threadIdx.x & 63, tap = threadIdx.x >> 6;
     const int ci0 = (int)blockIdx.x * 32, co0 = (int)blockIdx.y * 32;
     const int per_image = (h + rows - 1) / rows;
     const int pn = (int)blockIdx.z / per_image;
     const int r0 = ((int)blockIdx.z % per_image) * rows;
     const int r1 = r0 + rows < h ? r0 + rows : h;
+    // the chunk's lines and their positions, the pixels from one to the next
+    const int nl = TURN ? wd : r1 - r0, np = TURN ? r1 - r0 : wd;
+    const int ls = TURN ? 1 : wd, ps = TURN ? wd : 1;
+    const GradTile T = grad_tile(nl, np);
     // the chunk's rows of dout, and of the input with one around
     const int ya = r0 > 0 ? r0 - 1 : 0, yb = r1 < h ? r1 + 1 : h;
     const uint32_t xbytes = (uint32_t)(yb - ya) * (uint32_t)wd * (uint32_t)cin * 4u;
     const uint32_t dbytes = (uint32_t)(r1 - r0) * (uint32_t)wd * (uint32_t)cout * 4u;
     const __amdgpu_buffer_rsrc_t rx = buf(in + ((int64_t)pn * h + ya) * wd * cin, xbytes);
     const __amdgpu_buffer_rsrc_t rd = buf(dout + ((int64_t)pn * h + r0) * wd * cout, dbytes);
+    // the input's lines and positions, from the chunk's first
+    const int la = TURN ? 0 : ya - r0, lb = TURN ? wd : yb - r0;
+    const int pa = TURN ? ya - r0 : 0, pb = TURN ? yb - r0 : wd;
     const int xw = T.seg + 2;
     const FastDiv dseg = fast_div(T.seg), dxw = fast_div(xw);
     // staging items: 8 channels of a pixel; a thread keeps its channels
     constexpr int kX = (kGIn + NP - 1) / NP, kD = (kGPix + NP - 1) / NP;
     const int c8 = (int)threadIdx.x % 4 * 8, p0 = (int)threadIdx.x / 4;
     const int xleft = cin - ci0 - c8, dleft = cout - co0 - c8;
-    // the items' pixels in a sub-tile (rows past it: none), and their byte
+    // the items' pixels in a sub-tile (lines past it: none), and their byte
     // offsets from its first one
     int xty[kX], xtx[kX], dty[kD], dtx[kD];
     uint32_t xrel[kX], drel[kD];
@@ -432,42 +450,43 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
     for (int k = 0; k < kX; k++) {
         xty[k] = fdiv(p0 + k * NP, dxw, &xtx[k]) - 1;
         xtx[k]--;
-        xrel[k] = ((uint32_t)(xty[k] * wd + xtx[k]) * (uint32_t)cin + ci0 + c8) * 4u;
+        xrel[k] = ((uint32_t)(xty[k] * ls + xtx[k] * ps + (r0 - ya) * wd) * (uint32_t)cin + ci0 +
+                   c8) * 4u;
         if (xty[k] > T.rt) xty[k] = 1 << 30;
     }
 #pragma unroll
     for (int k = 0; k < kD; k++) {
         dty[k] = fdiv(p0 + k * NP, dseg, &dtx[k]);
-        drel[k] = ((uint32_t)(dty[k] * wd + dtx[k]) * (uint32_t)cout + co0 + c8) * 4u;
+        drel[k] = ((uint32_t)(dty[k] * ls + dtx[k] * ps) * (uint32_t)cout + co0 + c8) * 4u;
         if (dty[k] >= T.rt) dty[k] = 1 << 30;
     }
     float4 fx[kX][2], fd[kD][2];
-    // sub-tile: rows from ry, columns from cx
-    auto load = [&](int ry, int cx) {
-        const uint32_t xb = (uint32_t)((ry - ya) * wd + cx) * (uint32_t)cin * 4u;
-        const uint32_t db = (uint32_t)((ry - r0) * wd + cx) * (uint32_t)cout * 4u;
+    // sub-tile: lines from l, positions from p
+    auto load = [&](int l, int p) {
+        const uint32_t at = (uint32_t)(l * ls + p * ps);
+        const uint32_t xb = at * (uint32_t)cin * 4u, db = at * (uint32_t)cout * 4u;
 #pragma unroll
         for (int k = 0; k < kX; k++) {
-            const bool on = (uint32_t)(xty[k] + ry - ya) < (uint32_t)(yb - ya) &&
-                            (uint32_t)(xtx[k] + cx) < (uint32_t)wd;
+            const bool on = (uint32_t)(xty[k] + l - la) < (uint32_t)(lb - la) &&
+                            (uint32_t)(xtx[k] + p - pa) < (uint32_t)(pb - pa);
             load8<VEC>(fx[k], rx, xrel[k] + xb, on ? xleft : 0, xbytes);
         }
 #pragma unroll
         for (int k = 0; k < kD; k++) {
-            const bool on = dty[k] + ry < r1 && dtx[k] + cx < wd;
+            const bool on = dty[k] + l < nl && dtx[k] + p < np;
             load8<VEC>(fd[k], rd, drel[k] + db, on ? dleft : 0, dbytes);
         }
     };
     // this lane's part of a transposed read: group l / 16 reads channels
     // 16 (l / 16 % 2) .. and pixels 8 (l / 32) .. of a product's 16
     const int tr = (8 * (lane >> 5) + (lane & 15) / 4) * 32 + 16 * (lane >> 4 & 1) + 4 * (lane & 3);
-    const int shift = (tap / 3 * xw + tap % 3) * 32;
+    const int shift = (TURN ? tap % 3 * xw + tap / 3 : tap / 3 * xw + tap % 3) * 32;
     f32x16 acc = {};
     float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    load(r0, 0);
-    for (int ry = r0, cx = 0; ry < r1;) {
-        const int nx = cx + T.seg < wd ? cx + T.seg : 0, ny = nx ? ry : ry + T.rt;
-        if (ry > r0 || cx) __syncthreads();  // the products before have read
+    load(0, 0);
+    for (int ry = 0, cx = 0; ry < nl;) {
+        const int nx = cx + T.seg < np ? cx + T.seg : 0, ny = nx ? ry : ry + T.rt;
+        if (ry || cx) __syncthreads();  // the products before have read
 #pragma unroll
         for (int k = 0; k < kX; k++)
             if (p0 + k * NP < kGIn)
@@ -484,9 +503,9 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
             for (int c = 0; c < 8; c++) bsum[c] += v[c];
         }
         __syncthreads();
-        if (ny < r1) load(ny, nx);
-        const int nrows = r1 - ry < T.rt ? r1 - ry : T.rt;
-        // N products of a row, their reads ahead of them
+        if (ny < nl) load(ny, nx);
+        const int nrows = nl - ry < T.rt ? nl - ry : T.rt;
+        // N products of a line, their reads ahead of them
         auto products = [&](auto steps, const short* d, const short* x, int px) {
             constexpr int N = decltype(steps)::value;
             s16x8 a[N], b[N];
@@ -499,15 +518,15 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
                                                lds_tr(x + (px + 16 * i + 4) * 32), 0, 1, 2, 3, 4, 5,
                                                6, 7);
             }
-            // pixels past the row's end: their dout is zero, and so has to be
+            // pixels past the line's end: their dout is zero, and so has to be
             // the input beside it, whatever it holds
-            if (wd - cx - px < 16 * N) {
+            if (np - cx - px < 16 * N) {
 #pragma unroll
                 for (int i = 0; i < N; i++)
 #pragma unroll
                     for (int t = 0; t < 8; t++)
                         a[i][t] =
-                            px + 16 * i + 8 * (lane >> 5) + t < wd - cx ? a[i][t] : (short)0;
+                            px + 16 * i + 8 * (lane >> 5) + t < np - cx ? a[i][t] : (short)0;
             }
 #pragma unroll
             for (int i = 0; i < N; i++)
@@ -886,12 +905,14 @@ int mplbws_conv3x3_wgrad(const float* in, const float* dout, float* dw, float* d
     const int64_t cnt = (int64_t)K * cout;
     float* bp = dbias ? workspace + chunks * cnt : nullptr;
     const dim3 grd((unsigned)((cin + 31) / 32), (unsigned)((cout + 31) / 32), (unsigned)chunks);
-    if (vec4(in, dout, cin, cout, 0))
-        hipLaunchKernelGGL(k_conv_wgrad<true>, grd, dim3(64 * kGWaves), 0, 0, in, dout, workspace, bp,
-                           h, wd, cin, cout, rows);
-    else
-        hipLaunchKernelGGL(k_conv_wgrad<false>, grd, dim3(64 * kGWaves), 0, 0, in, dout, workspace,
-                           bp, h, wd, cin, cout, rows);
+    const bool turn = grad_tiles(wd, rows) < grad_tiles(rows, wd);
+    const bool vec = vec4(in, dout, cin, cout, 0);
+#define X(VEC, TURN)                                                                           \
+    if (vec == VEC && turn == TURN)                                                            \
+        hipLaunchKernelGGL((k_conv_wgrad<VEC, TURN>), grd, dim3(64 * kGWaves), 0, 0, in, dout, \
+                           workspace, bp, h, wd, cin, cout, rows);
+    X(true, false) X(true, true) X(false, false) X(false, true)
+#undef X
     const int64_t sums = (cnt + 63) / 64 + (dbias ? (cout + 63) / 64 : 0);
     hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)sums), dim3(64 * kSumWaves), 0, 0, workspace,
                        dw, cnt, bp, dbias, (int64_t)cout, (int)chunks);

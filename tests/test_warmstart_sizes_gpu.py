@@ -116,3 +116,49 @@ def test_convolution_of_few_rows(n, h, wd, cin, cout):
     # FP32 sums of 9 cin exact products
     tol = (9 * cin + 1) * 2.0 ** -24 * nno.conv3x3(np.abs(x), np.abs(w))
     assert (np.abs(out.numpy() - nno.conv3x3(x, w)) <= tol).all()
+
+
+# few columns (taken along them), two chunks of one and of nine, few rows in
+# long lines, and channel counts that are no multiple of four on either side
+@pytest.mark.parametrize("n,h,wd,cin,cout", [(1, 300, 1, 8, 4), (2, 130, 2, 5, 3), (1, 97, 3, 33, 12),
+                                             (3, 40, 7, 8, 67), (1, 5000, 1, 4, 4),
+                                             (1, 700, 9, 12, 8), (1, 1, 200, 8, 8),
+                                             (1, 2, 150, 6, 5), (2, 33, 33, 40, 35),
+                                             (2, 33, 33, 39, 36), (1, 20, 20, 1, 1)])
+def test_weight_gradient_of_thin_images_and_odd_channels(n, h, wd, cin, cout):
+    log("wgrad %s" % ((n, h, wd, cin, cout),))
+    lib, rng = ws.load(), np.random.default_rng(13)
+    A = ws.DeviceArray.from_numpy
+    x = rng.standard_normal((n, h, wd, cin)).astype(np.float32)
+    d = rng.standard_normal((n, h, wd, cout)).astype(np.float32)
+    dw, db = ws.DeviceArray((9, cin, cout)), ws.DeviceArray((cout,))
+    k = ws.DeviceArray((int(lib.mplbws_wgrad_workspace(n, h, wd, cin, cout)),))
+    ax, ad = A(x), A(d)
+    ck(lib.mplbws_conv3x3_wgrad(ax.p, ad.p, dw.p, db.p, k.p, n, h, wd, cin, cout))
+    ref, refb = nno.conv3x3_wgrad(x, d)
+    mag, magb = nno.conv3x3_wgrad(np.abs(x), np.abs(d))
+    # FP32 sums over the pixels
+    m = n * h * wd
+    assert (np.abs(dw.numpy() - ref) <= m * 2.0 ** -24 * mag).all()
+    assert (np.abs(db.numpy() - refb) <= m * 2.0 ** -24 * magb + 1e-30).all()
+
+
+def test_weight_gradient_drops_the_next_pixels_channels():
+    """With channel counts that are no multiple of four the loads are wider than
+    what is left of a pixel.  What they bring of another pixel is no part of a
+    sum, even where it is no number: here that pixel is behind the array, which
+    the rest of the allocation follows."""
+    lib, rng = ws.load(), np.random.default_rng(14)
+    n, h, wd, cin, cout = 1, 6, 21, 3, 5
+    x = rng.standard_normal((n, h, wd, cin)).astype(np.float32)
+    d = rng.standard_normal((n, h, wd, cout)).astype(np.float32)
+    nan = np.full(64, np.nan, np.float32)
+    ax = ws.DeviceArray.from_numpy(np.concatenate([nan, x.ravel(), nan]))
+    ad = ws.DeviceArray.from_numpy(np.concatenate([nan, d.ravel(), nan]))
+    dw, db = ws.DeviceArray((9, cin, cout)), ws.DeviceArray((cout,))
+    k = ws.DeviceArray((int(lib.mplbws_wgrad_workspace(n, h, wd, cin, cout)),))
+    ck(lib.mplbws_conv3x3_wgrad(at(ax, 64), at(ad, 64), dw.p, db.p, k.p, n, h, wd, cin, cout))
+    ref, _ = nno.conv3x3_wgrad(x, d)
+    mag, _ = nno.conv3x3_wgrad(np.abs(x), np.abs(d))
+    assert (np.abs(dw.numpy() - ref) <= n * h * wd * 2.0 ** -24 * mag).all()
+    assert np.isfinite(db.numpy()).all()
