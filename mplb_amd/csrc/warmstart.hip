@@ -114,6 +114,15 @@ __device__ __forceinline__ float buf_ld1(__amdgpu_buffer_rsrc_t r, uint32_t voff
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
+// 8 floats from p + off on, `left` of them real; zeros past them
+__device__ __forceinline__ void load8_wide(float4* f, const float* p, int64_t off, int left) {
+    float v[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) v[c] = left > c ? p[off + c] : 0.f;
+    f[0] = float4{v[0], v[1], v[2], v[3]};
+    f[1] = float4{v[4], v[5], v[6], v[7]};
+}
+
 // workgroups are dealt to the 8 XCDs in turn: consecutive tiles, which share
 // their halos, on one of them
 __device__ __forceinline__ int tile_order(int i, int count) {
@@ -121,9 +130,16 @@ __device__ __forceinline__ int tile_order(int i, int count) {
     return i < whole ? (i % 8) * per + i / 8 : i;
 }
 
-// VEC: cout is a multiple of four, and w and out are aligned for 16-byte
+// How a convolution addresses its operands: by buffer offsets of 32 bits, in
+// 16-byte accesses where channel counts and alignment allow them (kFormVec) or
+// not; by 64 bits (kFormWide) where a tile's rows, a chunk's or the weights are
+// 4 GiB and more.
+enum { kFormAny = 0, kFormVec = 1, kFormWide = 2 };
+template <int FORM> using Offset = std::conditional_t<FORM == kFormWide, int64_t, uint32_t>;
+
+// kFormVec: cout is a multiple of four, and w and out are aligned for 16-byte
 // accesses
-template <int WM, int WN, bool VEC>
+template <int WM, int WN, int FORM>
 __global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const float* __restrict__ in,
                                                           const float* __restrict__ w,
                                                           const float* __restrict__ bias,
@@ -131,6 +147,9 @@ __global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const
                                                           int h, int wd, int cin, int cout,
                                                           int relu) {
     constexpr int TP = 128 * WM, CG = 32 * WN, NT = 64 * kWaves;
+    constexpr bool WIDE = FORM == kFormWide, VEC = FORM == kFormVec;
+    using Off = Offset<FORM>;
+    constexpr Off unit = WIDE ? 1 : 4;  // offsets in floats, or in bytes
     __shared__ __attribute__((aligned(16))) short s_in[conv_max_staged(TP) * kPixStride];
     // A fragments: [tap][8 input channels][co 0 .. CG-1][8]
     __shared__ __attribute__((aligned(16))) short s_w[9 * (kCC / 8) * CG * 8];
@@ -167,9 +186,11 @@ __global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const
     constexpr int kIn = (conv_max_staged(TP) * (kCC / 8) + NT - 1) / NT;
     const int ya = y0 > 0 ? y0 - 1 : 0, yb = y0 + T.R + 1 < h ? y0 + T.R + 1 : h;
     const uint32_t ibytes = (uint32_t)(yb - ya) * (uint32_t)wd * (uint32_t)cin * 4u;
-    const __amdgpu_buffer_rsrc_t rin = buf(in + ((int64_t)pn * h + ya) * wd * cin, ibytes);
+    const float* rows_in = in + ((int64_t)pn * h + ya) * wd * cin;
+    const __amdgpu_buffer_rsrc_t rin = buf(rows_in, ibytes);
+    const Off inone = WIDE ? Off(-1) : Off(ibytes);
     const int c8 = (int)threadIdx.x & 3;
-    uint32_t ioff[kIn];
+    Off ioff[kIn];
 #pragma unroll
     for (int k = 0; k < kIn; k++) {
         const int sp = ((int)threadIdx.x + k * NT) >> 2;
@@ -177,21 +198,22 @@ __global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const
         const int sy = fdiv(sp, dsw, &sx);
         const int yy = y0 + sy - 1, xx = x0 + sx - 1;
         ioff[k] = sp < SP && yy >= 0 && yy < h && xx >= 0 && xx < wd
-                      ? ((uint32_t)((yy - ya) * wd + xx) * (uint32_t)cin + 8u * c8) * 4u
-                      : ibytes;
+                      ? (((Off)(yy - ya) * (Off)wd + (Off)xx) * (Off)cin + 8 * c8) * unit
+                      : inone;
     }
     // Weight item k: 8 input channels of one tap by 4 output channels.
     constexpr int kTot = 9 * (kCC / 8) * (CG / 4), kW = (kTot + NT - 1) / NT;
     const uint32_t wbytes = 9u * (uint32_t)cin * (uint32_t)cout * 4u;
     const __amdgpu_buffer_rsrc_t rw = buf(w, wbytes);
-    uint32_t woff[kW];
+    const Off wnone = WIDE ? Off(-1) : Off(wbytes);
+    Off woff[kW];
 #pragma unroll
     for (int k = 0; k < kW; k++) {
         const int e = (int)threadIdx.x + k * NT;
         const int oc = co0 + (e % (CG / 4)) * 4, j = e / (CG / 4);
         woff[k] = e < kTot && oc < cout
-                      ? (((uint32_t)(j >> 2) * cin + 8u * (j & 3)) * (uint32_t)cout + oc) * 4u
-                      : wbytes;
+                      ? (((Off)(j >> 2) * cin + 8 * (j & 3)) * (Off)cout + oc) * unit
+                      : wnone;
     }
     f32x16 acc[WM][WN] = {};
     for (int c0 = 0; c0 < cin; c0 += kCC) {
@@ -200,18 +222,29 @@ __global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const
         float4 f[kIn][2];
 #pragma unroll
         for (int k = 0; k < kIn; k++) {
-            const uint32_t off = 8 * c8 < cc ? ioff[k] : ibytes;
-            f[k][0] = buf_ld4(rin, off, c0 * 4u);
-            f[k][1] = buf_ld4(rin, off, c0 * 4u + 16u);
+            const Off off = 8 * c8 < cc ? ioff[k] : inone;
+            if constexpr (WIDE) {
+                load8_wide(f[k], rows_in, off + c0, off < 0 ? 0 : 8);
+            } else {
+                f[k][0] = buf_ld4(rin, off, c0 * 4u);
+                f[k][1] = buf_ld4(rin, off, c0 * 4u + 16u);
+            }
         }
         float4 u[8];
         auto load_w = [&](int k) {
             const int j = ((int)threadIdx.x + k * NT) / (CG / 4);
-            const uint32_t off = 8 * (j & 3) < cc ? woff[k] : wbytes;
+            const Off off = 8 * (j & 3) < cc ? woff[k] : wnone;
 #pragma unroll
             for (int r = 0; r < 8; r++) {
-                const uint32_t so = (uint32_t)(c0 + r) * (uint32_t)cout * 4u;
-                if constexpr (VEC) {
+                const Off so = (Off)(c0 + r) * (Off)cout * unit;
+                if constexpr (WIDE) {
+                    const int left = off < 0 ? 0 : cout - (int)(off % cout);
+                    const float* p = w + off + so;
+                    u[r].x = left > 0 ? p[0] : 0.f;
+                    u[r].y = left > 1 ? p[1] : 0.f;
+                    u[r].z = left > 2 ? p[2] : 0.f;
+                    u[r].w = left > 3 ? p[3] : 0.f;
+                } else if constexpr (VEC) {
                     u[r] = buf_ld4(rw, off, so);
                 } else {
                     const int left = off < wbytes ? cout - (int)((off / 4u) % (uint32_t)cout) : 0;
@@ -382,16 +415,16 @@ __device__ __forceinline__ s16x4 lds_tr(const short* p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
 }
 
-// 8 channels at a byte offset, `left` of them (a multiple of 4 if VEC) real;
-// zeros past them and for off = bytes.  Without VEC the loads are as wide, at
-// any multiple of four bytes, and what is not this pixel's is dropped (8
+// 8 channels at a byte offset, `left` of them (kFormVec: a multiple of 4) real;
+// zeros past them and for off = bytes.  kFormAny's loads are as wide, at any
+// multiple of four bytes, and what is not this pixel's is dropped (8
 // images of 64 x 64, 35 to 33 channels: 105 us by single floats, 48).
-template <bool VEC>
+template <int FORM>
 __device__ __forceinline__ void load8(float4* f, __amdgpu_buffer_rsrc_t r, uint32_t off, int left,
                                       uint32_t bytes) {
     f[0] = buf_ld4(r, left > 0 ? off : bytes, 0);
     f[1] = buf_ld4(r, left > 4 ? off + 16u : bytes, 0);
-    if constexpr (!VEC) {
+    if constexpr (FORM == kFormAny) {
         f[0].y = left > 1 ? f[0].y : 0.f;
         f[0].z = left > 2 ? f[0].z : 0.f;
         f[0].w = left > 3 ? f[0].w : 0.f;
@@ -401,12 +434,12 @@ __device__ __forceinline__ void load8(float4* f, __amdgpu_buffer_rsrc_t r, uint3
     }
 }
 
-// VEC: cin and cout are multiples of four, in and dout aligned for 16-byte
+// kFormVec: cin and cout are multiples of four, in and dout aligned for 16-byte
 // accesses.
 // TURN: where the chunk is in fewer sub-tiles by columns than by rows (1 x 4096
 // pixels by rows would be 256 sub-tiles of 16 columns each, one of them real:
 // 64 to 64 channels 1270 us, 55; 8 columns 166, 40).
-template <bool VEC, bool TURN>
+template <int FORM, bool TURN>
 __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __restrict__ in,
                                                                 const float* __restrict__ dout,
                                                                 float* __restrict__ partial,
@@ -414,6 +447,9 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
                                                                 int wd, int cin, int cout,
                                                                 int rows) {
     constexpr int NT = 64 * kGWaves, NP = NT / 4;
+    constexpr bool WIDE = FORM == kFormWide;
+    using Off = Offset<FORM>;
+    constexpr Off unit = WIDE ? 1 : 4;  // offsets in floats, or in bytes
     // [pixel][32 channels]
     __shared__ __attribute__((aligned(16))) short s_x[kGIn * 32];
     __shared__ __attribute__((aligned(16))) short s_d[kGPix * 32];
@@ -431,8 +467,9 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
     const int ya = r0 > 0 ? r0 - 1 : 0, yb = r1 < h ? r1 + 1 : h;
     const uint32_t xbytes = (uint32_t)(yb - ya) * (uint32_t)wd * (uint32_t)cin * 4u;
     const uint32_t dbytes = (uint32_t)(r1 - r0) * (uint32_t)wd * (uint32_t)cout * 4u;
-    const __amdgpu_buffer_rsrc_t rx = buf(in + ((int64_t)pn * h + ya) * wd * cin, xbytes);
-    const __amdgpu_buffer_rsrc_t rd = buf(dout + ((int64_t)pn * h + r0) * wd * cout, dbytes);
+    const float* px0 = in + ((int64_t)pn * h + ya) * wd * cin;
+    const float* pd0 = dout + ((int64_t)pn * h + r0) * wd * cout;
+    const __amdgpu_buffer_rsrc_t rx = buf(px0, xbytes), rd = buf(pd0, dbytes);
     // the input's lines and positions, from the chunk's first
     const int la = TURN ? 0 : ya - r0, lb = TURN ? wd : yb - r0;
     const int pa = TURN ? ya - r0 : 0, pb = TURN ? yb - r0 : wd;
@@ -445,36 +482,38 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
     // the items' pixels in a sub-tile (lines past it: none), and their byte
     // offsets from its first one
     int xty[kX], xtx[kX], dty[kD], dtx[kD];
-    uint32_t xrel[kX], drel[kD];
+    Off xrel[kX], drel[kD];
 #pragma unroll
     for (int k = 0; k < kX; k++) {
         xty[k] = fdiv(p0 + k * NP, dxw, &xtx[k]) - 1;
         xtx[k]--;
-        xrel[k] = ((uint32_t)(xty[k] * ls + xtx[k] * ps + (r0 - ya) * wd) * (uint32_t)cin + ci0 +
-                   c8) * 4u;
+        xrel[k] = (((Off)xty[k] * (Off)ls + (Off)xtx[k] * (Off)ps + (Off)(r0 - ya) * (Off)wd) *
+                       (Off)cin + ci0 + c8) * unit;
         if (xty[k] > T.rt) xty[k] = 1 << 30;
     }
 #pragma unroll
     for (int k = 0; k < kD; k++) {
         dty[k] = fdiv(p0 + k * NP, dseg, &dtx[k]);
-        drel[k] = ((uint32_t)(dty[k] * ls + dtx[k] * ps) * (uint32_t)cout + co0 + c8) * 4u;
+        drel[k] = (((Off)dty[k] * (Off)ls + (Off)dtx[k] * (Off)ps) * (Off)cout + co0 + c8) * unit;
         if (dty[k] >= T.rt) dty[k] = 1 << 30;
     }
     float4 fx[kX][2], fd[kD][2];
     // sub-tile: lines from l, positions from p
     auto load = [&](int l, int p) {
-        const uint32_t at = (uint32_t)(l * ls + p * ps);
-        const uint32_t xb = at * (uint32_t)cin * 4u, db = at * (uint32_t)cout * 4u;
+        const Off at = (Off)l * (Off)ls + (Off)p * (Off)ps;
+        const Off xb = at * (Off)cin * unit, db = at * (Off)cout * unit;
 #pragma unroll
         for (int k = 0; k < kX; k++) {
             const bool on = (uint32_t)(xty[k] + l - la) < (uint32_t)(lb - la) &&
                             (uint32_t)(xtx[k] + p - pa) < (uint32_t)(pb - pa);
-            load8<VEC>(fx[k], rx, xrel[k] + xb, on ? xleft : 0, xbytes);
+            if constexpr (WIDE) load8_wide(fx[k], px0, xrel[k] + xb, on ? xleft : 0);
+            else load8<FORM>(fx[k], rx, xrel[k] + xb, on ? xleft : 0, xbytes);
         }
 #pragma unroll
         for (int k = 0; k < kD; k++) {
             const bool on = dty[k] + l < nl && dtx[k] + p < np;
-            load8<VEC>(fd[k], rd, drel[k] + db, on ? dleft : 0, dbytes);
+            if constexpr (WIDE) load8_wide(fd[k], pd0, drel[k] + db, on ? dleft : 0);
+            else load8<FORM>(fd[k], rd, drel[k] + db, on ? dleft : 0, dbytes);
         }
     };
     // this lane's part of a transposed read: group l / 16 reads channels
@@ -857,22 +896,18 @@ int mplbws_conv3x3_fwd(const float* in, const float* w, const float* bias, float
     const int wm = (int64_t)n * T2.tiles_x * T2.tiles_y * groups >= 512 ? 2 : 1;
     const ConvTile T = conv_tile(h, wd, 128 * wm);
     const int64_t wgs = (int64_t)n * T.tiles_x * T.tiles_y;
-    // (a tile's rows and the weights are addressed by 32-bit offsets)
-    if (wgs >= ((int64_t)1 << 31) || (int64_t)(T.R + 2) * wd * cin >= (int64_t)1 << 30 ||
-        9LL * cin * cout >= (int64_t)1 << 30)
-        return MPLBWS_ERR_ARG;
+    if (wgs >= ((int64_t)1 << 31)) return MPLBWS_ERR_ARG;
     const dim3 grd((unsigned)wgs, (unsigned)groups), blk(64 * kWaves);
-    const bool vec = vec4(w, out, cout, 0, 0);
-#define X(WM, WN)                                                                             \
-    if (wm == WM && wn == WN) {                                                               \
-        if (vec)                                                                              \
-            hipLaunchKernelGGL((k_conv_fwd<WM, WN, true>), grd, blk, 0, 0, in, w, bias, out, n, \
-                               h, wd, cin, cout, relu);                                       \
-        else                                                                                  \
-            hipLaunchKernelGGL((k_conv_fwd<WM, WN, false>), grd, blk, 0, 0, in, w, bias, out, n, \
-                               h, wd, cin, cout, relu);                                       \
-    }
-    X(2, 2) X(2, 1) X(1, 2) X(1, 1)
+    const bool wide = (int64_t)(T.R + 2) * wd >= (((int64_t)1 << 30) + cin - 1) / cin ||
+                      9LL * cin * cout >= (int64_t)1 << 30;
+    const int form = wide ? kFormWide : vec4(w, out, cout, 0, 0) ? kFormVec : kFormAny;
+#define X(WM, WN, FORM)                                                                        \
+    if (wm == WM && wn == WN && form == FORM)                                                  \
+        hipLaunchKernelGGL((k_conv_fwd<WM, WN, FORM>), grd, blk, 0, 0, in, w, bias, out, n, h, \
+                           wd, cin, cout, relu);
+    X(2, 2, kFormAny) X(2, 1, kFormAny) X(1, 2, kFormAny) X(1, 1, kFormAny)
+    X(2, 2, kFormVec) X(2, 1, kFormVec) X(1, 2, kFormVec) X(1, 1, kFormVec)
+    X(2, 2, kFormWide) X(2, 1, kFormWide) X(1, 2, kFormWide) X(1, 1, kFormWide)
 #undef X
     return status();
 }
@@ -898,20 +933,21 @@ int mplbws_conv3x3_wgrad(const float* in, const float* dout, float* dw, float* d
         return MPLBWS_ERR_ARG;
     const int rows = wgrad_rows(h, wd);
     const int64_t chunks = (int64_t)n * ((h + rows - 1) / rows);
-    // (a chunk's rows are addressed by 32-bit offsets)
-    if (chunks > 65535 || (int64_t)(rows + 2) * wd * std::max(cin, cout) >= (int64_t)1 << 30)
-        return MPLBWS_ERR_ARG;
+    if (chunks > 65535) return MPLBWS_ERR_ARG;
     const int K = 9 * cin;
     const int64_t cnt = (int64_t)K * cout;
     float* bp = dbias ? workspace + chunks * cnt : nullptr;
     const dim3 grd((unsigned)((cin + 31) / 32), (unsigned)((cout + 31) / 32), (unsigned)chunks);
     const bool turn = grad_tiles(wd, rows) < grad_tiles(rows, wd);
-    const bool vec = vec4(in, dout, cin, cout, 0);
-#define X(VEC, TURN)                                                                           \
-    if (vec == VEC && turn == TURN)                                                            \
-        hipLaunchKernelGGL((k_conv_wgrad<VEC, TURN>), grd, dim3(64 * kGWaves), 0, 0, in, dout, \
+    const int64_t most = std::max(cin, cout);
+    const bool wide = (int64_t)(rows + 2) * wd >= (((int64_t)1 << 30) + most - 1) / most;
+    const int form = wide ? kFormWide : vec4(in, dout, cin, cout, 0) ? kFormVec : kFormAny;
+#define X(FORM, TURN)                                                                           \
+    if (form == FORM && turn == TURN)                                                           \
+        hipLaunchKernelGGL((k_conv_wgrad<FORM, TURN>), grd, dim3(64 * kGWaves), 0, 0, in, dout, \
                            workspace, bp, h, wd, cin, cout, rows);
-    X(true, false) X(true, true) X(false, false) X(false, true)
+    X(kFormAny, false) X(kFormVec, false) X(kFormWide, false)
+    X(kFormAny, true) X(kFormVec, true) X(kFormWide, true)
 #undef X
     const int64_t sums = (cnt + 63) / 64 + (dbias ? (cout + 63) / 64 : 0);
     hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)sums), dim3(64 * kSumWaves), 0, 0, workspace,

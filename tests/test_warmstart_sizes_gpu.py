@@ -162,3 +162,66 @@ def test_weight_gradient_drops_the_next_pixels_channels():
     mag, _ = nno.conv3x3_wgrad(np.abs(x), np.abs(d))
     assert (np.abs(dw.numpy() - ref) <= n * h * wd * 2.0 ** -24 * mag).all()
     assert np.isfinite(db.numpy()).all()
+
+
+def _patches(lib, d, width, channels, starts, rng):
+    """A zeroed array of `width` pixels with 40 random ones from each start on."""
+    ck(lib.mplbws_zero(d.p, 4 * d.numel()))
+    out = []
+    for s in starts:
+        a = rng.standard_normal((1, 1, 40, channels)).astype(np.float32)
+        ck(lib.mplbws_upload(at(d, s * channels), a.ctypes.data, a.nbytes))
+        out.append(a)
+    return out
+
+
+def test_convolution_of_rows_past_four_gib():
+    """One row of 2^20 pixels x 1040 channels (4.4 GB), zero but for a few
+    patches, one of them past the 32-bit offsets and at the row's end."""
+    lib, rng = ws.load(), np.random.default_rng(15)
+    wd, cin, cout = 1 << 20, 1040, 5
+    starts = (0, 500001, wd - 40)
+    assert (wd - 40) * cin * 4 > 1 << 32
+    x, out = ws.DeviceArray((wd, cin)), ws.DeviceArray((wd, cout))
+    patches = _patches(lib, x, wd, cin, starts, rng)
+    w = (rng.standard_normal((9, cin, cout)) / 8).astype(np.float32)
+    dw = ws.DeviceArray.from_numpy(w)
+    ck(lib.mplbws_conv3x3_fwd(x.p, dw.p, None, out.p, 1, 1, wd, cin, cout, 0))
+    got = out.numpy()
+    for s, a in zip(starts, patches):
+        mag = (9 * cin + 1) * 2.0 ** -24 * nno.conv3x3(np.abs(a), np.abs(w))[0, 0]
+        assert (np.abs(got[s:s + 40] - nno.conv3x3(a, w)[0, 0]) <= mag).all(), s
+    assert not got[41:500000].any() and not got[500042:wd - 41].any()
+
+
+def test_convolution_of_weights_past_four_gib():
+    lib, rng = ws.load(), np.random.default_rng(16)
+    cin, cout = 10928, 10930
+    assert 9 * cin * cout * 4 > 1 << 32
+    x = rng.standard_normal((1, 1, 2, cin)).astype(np.float32)
+    w = np.resize(rng.standard_normal(1000003).astype(np.float32), (9, cin, cout))
+    dx, dw, out = ws.DeviceArray.from_numpy(x), ws.DeviceArray.from_numpy(w), ws.DeviceArray((2, cout))
+    ck(lib.mplbws_conv3x3_fwd(dx.p, dw.p, None, out.p, 1, 1, 2, cin, cout, 0))
+    some = np.r_[0:3, 5000:5003, cout - 3:cout]
+    ws_ = np.ascontiguousarray(w[:, :, some])
+    tol = (9 * cin + 1) * 2.0 ** -24 * nno.conv3x3(np.abs(x), np.abs(ws_))[0, 0]
+    assert (np.abs(out.numpy()[:, some] - nno.conv3x3(x, ws_)[0, 0]) <= tol).all()
+
+
+def test_weight_gradient_of_rows_past_four_gib():
+    lib, rng = ws.load(), np.random.default_rng(17)
+    wd, cin, cout = 1 << 20, 3, 1040
+    starts = (0, 500001, wd - 40)
+    x, d = ws.DeviceArray((wd, cin)), ws.DeviceArray((wd, cout))
+    xs, ds = (_patches(lib, a, wd, c, starts, rng) for a, c in ((x, cin), (d, cout)))
+    dw, db = ws.DeviceArray((9, cin, cout)), ws.DeviceArray((cout,))
+    k = ws.DeviceArray((int(lib.mplbws_wgrad_workspace(1, 1, wd, cin, cout)),))
+    ck(lib.mplbws_conv3x3_wgrad(x.p, d.p, dw.p, db.p, k.p, 1, 1, wd, cin, cout))
+    ref, refb, mag, magb = 0, 0, 0, 0
+    for a, b in zip(xs, ds):
+        r, rb = nno.conv3x3_wgrad(a, b)
+        m, mb = nno.conv3x3_wgrad(np.abs(a), np.abs(b))
+        ref, refb, mag, magb = ref + r, refb + rb, mag + m, magb + mb
+    # FP32 sums of 120 terms that are not zero
+    assert (np.abs(dw.numpy() - ref) <= 120 * 2.0 ** -24 * mag).all()
+    assert (np.abs(db.numpy() - refb) <= 120 * 2.0 ** -24 * magb + 1e-30).all()
