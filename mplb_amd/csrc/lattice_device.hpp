@@ -162,15 +162,42 @@ template <typename OP> __device__ __forceinline__ float eq_coef(const OP& op, in
     return op.fcq[q];
 }
 
+// v where bit q of m is set, else +0; a where it is set, else b: exact
+// whatever they hold
+__device__ __forceinline__ float bit_and(float v, uint32_t m, int q) {
+    return __uint_as_float(__float_as_uint(v) & (uint32_t)((int32_t)(m << (31 - q)) >> 31));
+}
+__device__ __forceinline__ double bit_and(double v, uint32_t m, int q) {
+    const int64_t k = (int32_t)(m << (31 - q)) >> 31;
+    return __builtin_bit_cast(double, __builtin_bit_cast(int64_t, v) & k);
+}
+__device__ __forceinline__ float bit_or(float a, float b) {
+    return __uint_as_float(__float_as_uint(a) | __float_as_uint(b));
+}
+__device__ __forceinline__ double bit_or(double a, double b) {
+    return __builtin_bit_cast(double,
+                              __builtin_bit_cast(int64_t, a) | __builtin_bit_cast(int64_t, b));
+}
+__device__ __forceinline__ float bit_sel(uint32_t m, int q, float a, float b) {
+    const uint32_t k = (uint32_t)((int32_t)(m << (31 - q)) >> 31);
+    return __uint_as_float((__float_as_uint(a) & k) | (__float_as_uint(b) & ~k));
+}
+__device__ __forceinline__ double bit_sel(uint32_t m, int q, double a, double b) {
+    const int64_t k = (int32_t)(m << (31 - q)) >> 31;
+    return __builtin_bit_cast(double, (__builtin_bit_cast(int64_t, a) & k) |
+                                          (__builtin_bit_cast(int64_t, b) & ~k));
+}
+
 // KerCutCellEQMDiffuseRefl[3D] (boundary_kernel.inc:534-613, 1184-1276).
 // With the wall-velocity terms from the host (BCOp::den, cq): rho_w = 2
 // sum_in f / den, a parallel population (w rho_w) res, an outgoing one f_opp
-// + (w rho_w) (2 cu).  Every rounding is the reference's: a factor two, a
-// factor zero or one and an added zero are exact, so the classes are chosen
-// by multiply-adds with uniform 0/1 factors (scalar selects) and the code
-// has no branch.  With a scalar branch per population and class an
-// application took some 60 branches and as many dependent scalar loads,
-// which set the pace of every workgroup that waits for its wall lanes.
+// + (w rho_w) (2 cu).  Every rounding is the reference's: a factor two and an
+// added zero are exact.  The classes are chosen by bit masks, so the code has
+// no branch, and only incoming populations are read, so that no other one,
+// finite or not, has a part in the result.  With a scalar branch per
+// population and class an application took some 60 branches and as many
+// dependent scalar loads, which set the pace of every workgroup that waits
+// for its wall lanes.
 template <int D, typename T, typename OP>
 __device__ __forceinline__ void apply_eqm(T* f, const OP& op) {
 #pragma clang fp contract(off)
@@ -178,19 +205,17 @@ __device__ __forceinline__ void apply_eqm(T* f, const OP& op) {
     const uint32_t m_in = op.m_in, m_out = op.m_out, m_set = op.m_out | op.m_par;
     T rin = T(0);
 #pragma unroll
-    for (int q = 0; q < Q; q++) rin = fma_t(f[q], (m_in >> q & 1u) ? T(1) : T(0), rin);
+    for (int q = 0; q < Q; q++) rin += bit_and(f[q], m_in, q);
     const T rw = T(2) * rin / eq_den(op, T(0));
 #pragma unroll
     for (int q = 0; q < Q; q++) {
         const int p = opp(D, q);
         if (p < q) continue;
         const T wr = T(wgt(D, q)) * rw;
-        const T bq = fma_t(f[p], (m_out >> q & 1u) ? T(1) : T(0),
-                           f[q] * ((m_set >> q & 1u) ? T(0) : T(1)));
-        const T bp = fma_t(f[q], (m_out >> p & 1u) ? T(1) : T(0),
-                           f[p] * ((m_set >> p & 1u) ? T(0) : T(1)));
-        f[q] = wr * eq_coef(op, q, T(0)) + bq;
-        if (p != q) f[p] = wr * eq_coef(op, p, T(0)) + bp;
+        const T vq = wr * eq_coef(op, q, T(0)) + bit_and(f[p], m_out, q);
+        const T vp = wr * eq_coef(op, p, T(0)) + bit_and(f[q], m_out, p);
+        f[q] = bit_sel(m_set, q, vq, f[q]);
+        if (p != q) f[p] = bit_sel(m_set, p, vp, f[p]);
     }
 }
 
@@ -198,28 +223,26 @@ __device__ __forceinline__ void apply_eqm(T* f, const OP& op) {
 // with the terms that depend on the wall velocity only computed by the
 // host (BCOp::eq_*): rho_in = sum_in w + sum_in g, rho_w = 2 rho_in /
 // (1 - dRho - rhoPar), parallel g = rho_w w res - w, outgoing g = g_opp +
-// 2 rho_w w c.u (the w of a population and its opposite are equal); the
-// classes as 0/1 factors
+// 2 rho_w w c.u (the w of a population and its opposite are equal)
 template <int D, typename OP>
 __device__ __forceinline__ void apply_eqm_dev(float* g, const OP& op) {
     constexpr int Q = lq(D);
     const uint32_t m_in = op.m_in, m_out = op.m_out, m_par = op.m_par, m_set = m_out | m_par;
     float rin = op.eq_win;
 #pragma unroll
-    for (int q = 0; q < Q; q++) rin = __builtin_fmaf(g[q], (m_in >> q & 1u) ? 1.f : 0.f, rin);
+    for (int q = 0; q < Q; q++) rin += bit_and(g[q], m_in, q);
     const float rw = rin * op.eq_k;
-    auto base = [&](int q, int p) {
-        const float t = __builtin_fmaf(g[q], (m_set >> q & 1u) ? 0.f : 1.f,
-                                       (m_par >> q & 1u) ? -float(wgt(D, q)) : 0.f);
-        return __builtin_fmaf(g[p], (m_out >> q & 1u) ? 1.f : 0.f, t);
+    auto value = [&](int q, int p) {
+        const float b = bit_or(bit_and(g[p], m_out, q), bit_and(-float(wgt(D, q)), m_par, q));
+        return __builtin_fmaf(rw, op.eq_c[q], b);
     };
 #pragma unroll
     for (int q = 0; q < Q; q++) {
         const int p = opp(D, q);
         if (p < q) continue;
-        const float bq = base(q, p), bp = base(p, q);
-        g[q] = __builtin_fmaf(rw, op.eq_c[q], bq);
-        if (p != q) g[p] = __builtin_fmaf(rw, op.eq_c[p], bp);
+        const float vq = value(q, p), vp = value(p, q);
+        g[q] = bit_sel(m_set, q, vq, g[q]);
+        if (p != q) g[p] = bit_sel(m_set, p, vp, g[p]);
     }
 }
 

@@ -69,22 +69,6 @@ __device__ void load_walls(PairWalls<D, typename Store<ST>::T>& W, const RegionP
     }
 }
 
-// v where bit q of m is set, else +0: exact whatever v holds
-__device__ __forceinline__ float bit_and(float v, uint32_t m, int q) {
-    return __uint_as_float(__float_as_uint(v) & (uint32_t)((int32_t)(m << (31 - q)) >> 31));
-}
-__device__ __forceinline__ double bit_and(double v, uint32_t m, int q) {
-    const int64_t k = (int32_t)(m << (31 - q)) >> 31;
-    return __builtin_bit_cast(double, __builtin_bit_cast(int64_t, v) & k);
-}
-__device__ __forceinline__ float bit_or(float a, float b) {
-    return __uint_as_float(__float_as_uint(a) | __float_as_uint(b));
-}
-__device__ __forceinline__ double bit_or(double a, double b) {
-    return __builtin_bit_cast(double,
-                              __builtin_bit_cast(int64_t, a) | __builtin_bit_cast(int64_t, b));
-}
-
 // pair_boundary of a face or edge whose populations' classes are known at
 // compile time: the faces, and the edges that every plane has.  The general
 // form issues about 350 instructions; one wave per tile runs it while the
@@ -132,7 +116,7 @@ __device__ __forceinline__ void pair_boundary(PairWalls<D, typename Store<ST>::T
         if (wall) {
             const int s = r;
             const uint32_t m_in = W.mask[s][0], m_out = W.mask[s][1], m_par = W.mask[s][2];
-            const uint32_t keep = ~(m_out | m_par);
+            const uint32_t m_set = m_out | m_par;
             T rin = W.win[s];
 #pragma unroll
             for (int q = 0; q < Q; q++) rin += bit_and(f[q], m_in, q);
@@ -141,12 +125,11 @@ __device__ __forceinline__ void pair_boundary(PairWalls<D, typename Store<ST>::T
             for (int q = 0; q < Q; q++) {
                 const int p = opp(D, q);
                 if (p < q) continue;
-                const T bq = bit_or(bit_or(bit_and(f[q], keep, q), bit_and(f[p], m_out, q)),
-                                    bit_and(-T(wgt(D, q)), m_par, q));
-                const T bp = bit_or(bit_or(bit_and(f[p], keep, p), bit_and(f[q], m_out, p)),
-                                    bit_and(-T(wgt(D, p)), m_par, p));
-                f[q] = fma_t(rw, W.c[s][q], bq);
-                if (p != q) f[p] = fma_t(rw, W.c[s][p], bp);
+                const T bq = bit_or(bit_and(f[p], m_out, q), bit_and(-T(wgt(D, q)), m_par, q));
+                const T bp = bit_or(bit_and(f[q], m_out, p), bit_and(-T(wgt(D, p)), m_par, p));
+                const T vq = fma_t(rw, W.c[s][q], bq), vp = fma_t(rw, W.c[s][p], bp);
+                f[q] = bit_sel(m_set, q, vq, f[q]);
+                if (p != q) f[p] = bit_sel(m_set, p, vp, f[p]);
             }
         }
         return;
@@ -166,7 +149,7 @@ __device__ __forceinline__ void pair_boundary(PairWalls<D, typename Store<ST>::T
     if (wall) {
         const int s = r;
         const uint32_t m_in = W.mask[s][0], m_out = W.mask[s][1];
-        const uint32_t keep = ~(m_out | W.mask[s][2]);
+        const uint32_t m_set = m_out | W.mask[s][2];
         T rin = T(0);
 #pragma unroll
         for (int q = 0; q < Q; q++) rin += bit_and(f[q], m_in, q);
@@ -176,10 +159,10 @@ __device__ __forceinline__ void pair_boundary(PairWalls<D, typename Store<ST>::T
             const int p = opp(D, q);
             if (p < q) continue;
             const T wr = T(wgt(D, q)) * rw;
-            const T bq = bit_or(bit_and(f[q], keep, q), bit_and(f[p], m_out, q));
-            const T bp = bit_or(bit_and(f[p], keep, p), bit_and(f[q], m_out, p));
-            f[q] = wr * W.c[s][q] + bq;
-            if (p != q) f[p] = wr * W.c[s][p] + bp;
+            const T vq = wr * W.c[s][q] + bit_and(f[p], m_out, q);
+            const T vp = wr * W.c[s][p] + bit_and(f[q], m_out, p);
+            f[q] = bit_sel(m_set, q, vq, f[q]);
+            if (p != q) f[p] = bit_sel(m_set, p, vp, f[p]);
         }
     }
     if (persist >= 0 && own) {
