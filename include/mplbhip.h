@@ -161,8 +161,8 @@ int mplbhip_step_timed(mplbhip_ctx* ctx, int nsteps, double* ms_total,
  * shares of the last mplbhip_step_timed call (ms, summed over its steps). */
 int mplbhip_kernel_times(mplbhip_ctx* ctx, double* ms_bulk, double* ms_boundary);
 /* Diagnostic, no reference counterpart: the single-step launch shape in force
- * (after its autotuning: the first step, or where two steps share a launch
- * the first timed run or the 65th step taken singly): fold level (0 none, 1 simple x faces,
+ * (after its autotuning: the first step, or where several steps share a
+ * launch the 65th step taken singly): fold level (0 none, 1 simple x faces,
  * 2 every simple region of the planes z = 1 .. n-2, 3 every simple region
  * of every plane, 3D only; MPLBHIP_XFACE_FOLD fixes it), bulk workgroup
  * shape (0 plain tiles, 1 rows dealt to one XCD, 2 row workgroups), 1 if

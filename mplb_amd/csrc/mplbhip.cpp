@@ -2063,12 +2063,13 @@ int mplbhip_set_accel(mplbhip_ctx* c, int block, const double* g) {
     return 0;
 }
 
-// Launch-configuration autotuning, once per context on its first step:
-// which simple boundary regions the bulk kernel runs inline (none, the x
-// faces, all of its grid's), and keeping a row's tiles on one XCD or not.  Each candidate runs the step kernels a
-// few times from the current state into the other buffer; those writes are
-// what the next real step writes again, so the state is unchanged.  Cases
-// under 2^20 nodes keep the defaults (their steps are launch-bound).
+// Launch-configuration autotuning, once per context: which simple boundary
+// regions the bulk kernel runs inline (none, the x faces, all of its grid's),
+// and keeping a row's tiles on one XCD or not.  Each candidate runs the step
+// kernels a few times from the current state into the other buffer, which
+// holds the step before the latest, that macros and f are re-streamed from: a
+// real single step has to follow, whose writes replace those.  Cases under
+// 2^20 nodes keep the defaults (their steps are launch-bound).
 static int autotune(mplbhip_ctx* c) {
     if (c->tuned) return 0;
     c->tuned = true;
@@ -2135,6 +2136,15 @@ static int autotune(mplbhip_ctx* c) {
         std::fprintf(stderr, "mplbhip: autotune picked fold=%d xgroup=%d h2=%d (%.4f ms/step)\n",
                      c->fold, c->xgroup, (int)c->h2, best);
     return 0;
+}
+
+// The tuning, ahead of a single step of the stream-collision scheme over every
+// block: at once where single steps are what runs; beside launches of several
+// steps, where single ones only end a run, from the 65th on.
+static int tune_single(mplbhip_ctx* c) {
+    if (c->tuned || c->swap || c->grid_nodes != c->interior_nodes) return 0;
+    if (launch_steps(c) > 1 && ++c->singles <= 64) return 0;
+    return autotune(c);
 }
 
 // the swap scheme's f^0 in its one lattice: feq of the initial macros, or
@@ -2207,7 +2217,8 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         if (int rc = first_collision(c)) return rc;
     double ktot = 0.0;
     if (timed) {
-        if (int rc = autotune(c)) return rc;
+        if (nsteps > 0)
+            if (int rc = tune_single(c)) return rc;
         if (int rc = fresh_halos(c)) return rc;
         // per-step events bracket the bulk kernel and the boundary kernel,
         // each on the stream it runs on (the step's own launch structure)
@@ -2301,9 +2312,7 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
         left -= n;
     }
     while (left > 0) {
-        // a program that takes its steps one at a time gets them tuned too
-        if (ls > 1 && !c->tuned && ++c->singles > 64)
-            if (int rc = autotune(c)) return rc;
+        if (int rc = tune_single(c)) return rc;
         if (int rc = enqueue_step(c, false, false)) return rc;
         c->tstep++;
         left--;
@@ -2341,6 +2350,7 @@ int mplbhip_iterate(mplbhip_ctx* c, double criteria, int check_period,
         if (done >= max_steps) break;
         if (c->tstep == 0)
             if (int rc = first_collision(c)) return rc;
+        if (int rc = tune_single(c)) return rc;
         if (int rc = enqueue_step(c, true, converge)) return rc;
         c->tstep++;
         done++;
@@ -2528,6 +2538,7 @@ int mplbhip_iterate_batch(mplbhip_ctx* c, double criteria, int check_period,
         if (done >= max_steps) break;
         if (c->tstep == 0)
             if (int rc = first_collision(c)) return rc;
+        if (int rc = tune_single(c)) return rc;
         if (int rc = enqueue_step(c, true, true)) return rc;
         c->tstep++;
         done++;
