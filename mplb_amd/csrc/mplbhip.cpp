@@ -2140,10 +2140,14 @@ static int autotune(mplbhip_ctx* c) {
 
 // The tuning, ahead of a single step of the stream-collision scheme over every
 // block: at once where single steps are what runs; beside launches of several
-// steps, where single ones only end a run, from the 65th on.
-static int tune_single(mplbhip_ctx* c) {
+// steps, where single ones only end a run, from the 65th on.  period: a check
+// step's, which counts if no launch of several steps fits before it (else one
+// step in hundreds is single: at 256^3 tuning takes 0.1 s, for at most 0.02 ms
+// of each).
+static int tune_single(mplbhip_ctx* c, int period = 0) {
     if (c->tuned || c->swap || c->grid_nodes != c->interior_nodes) return 0;
-    if (launch_steps(c) > 1 && ++c->singles <= 64) return 0;
+    const int ls = launch_steps(c);
+    if (ls > 1 && (period > ls || ++c->singles <= 64)) return 0;
     return autotune(c);
 }
 
@@ -2350,7 +2354,7 @@ int mplbhip_iterate(mplbhip_ctx* c, double criteria, int check_period,
         if (done >= max_steps) break;
         if (c->tstep == 0)
             if (int rc = first_collision(c)) return rc;
-        if (int rc = tune_single(c)) return rc;
+        if (int rc = tune_single(c, check_period)) return rc;
         if (int rc = enqueue_step(c, true, converge)) return rc;
         c->tstep++;
         done++;
@@ -2538,7 +2542,7 @@ int mplbhip_iterate_batch(mplbhip_ctx* c, double criteria, int check_period,
         if (done >= max_steps) break;
         if (c->tstep == 0)
             if (int rc = first_collision(c)) return rc;
-        if (int rc = tune_single(c)) return rc;
+        if (int rc = tune_single(c, check_period)) return rc;
         if (int rc = enqueue_step(c, true, true)) return rc;
         c->tstep++;
         done++;
