@@ -170,6 +170,16 @@ int mplbhip_kernel_times(mplbhip_ctx* ctx, double* ms_bulk, double* ms_boundary)
  * updates (interior nodes plus the folded boundary nodes). */
 int mplbhip_launch_shape(mplbhip_ctx* ctx, int* fold, int* xgroup, int* h2,
                          long long* bulk_nodes);
+/* Diagnostic, no reference counterpart: what mplbhip_step launches for the
+ * case as it is defined now -- the kernel form and the steps of one launch at
+ * most.  A run of launches of several steps ends with a single step, which
+ * macros and f are measured from. */
+#define MPLBHIP_FORM_SINGLE 0 /* a step per launch (or bulk and boundary kernels) */
+#define MPLBHIP_FORM_PAIR 1   /* two steps of 3D blocks of walls */
+#define MPLBHIP_FORM_TILE 2   /* several steps of 2D blocks, in tiles */
+#define MPLBHIP_FORM_MARCH 3  /* several steps of 2D blocks, row by row */
+#define MPLBHIP_FORM_SWAP 4   /* the swap scheme in one pass per step */
+int mplbhip_step_form(mplbhip_ctx* ctx, int* form, int* steps);
 /* Iterate (evolution.cpp:71-135 and the templates evolution.h:78-129).
  * criteria < 0: run exactly max_steps steps, refreshing the macro variables
  * at every check_period-th step (the transient form).  criteria >= 0: step

@@ -2706,6 +2706,21 @@ int mplbhip_launch_shape(mplbhip_ctx* c, int* fold, int* xgroup, int* h2,
     return 0;
 }
 
+int mplbhip_step_form(mplbhip_ctx* c, int* form, int* steps) {
+    if (!c) return MPLBHIP_ERR_ARG;
+    if (int rc = need_device(c)) return rc;
+    if (!c->prepared) return fail(c, MPLBHIP_ERR_ARG, "call mplbhip_prepare first");
+    const int ls = launch_steps(c);
+    if (form)
+        *form = c->swap_pull ? MPLBHIP_FORM_SWAP
+                : ls == 1    ? MPLBHIP_FORM_SINGLE
+                : c->tile    ? MPLBHIP_FORM_TILE
+                : c->pair    ? MPLBHIP_FORM_PAIR
+                             : MPLBHIP_FORM_MARCH;
+    if (steps) *steps = ls;
+    return 0;
+}
+
 int mplbhip_update_macros(mplbhip_ctx* c) {
     if (!c) return MPLBHIP_ERR_ARG;
     if (int rc = need_device(c)) return rc;

@@ -19,6 +19,7 @@ LIB_PATH = os.path.join(_HERE, "libmplbhip.so")
 HEADER = os.path.join(os.path.dirname(_HERE), "include", "mplbhip.h")
 
 STORE_F64, STORE_F32, STORE_F16 = 0, 1, 2
+STEP_FORMS = ("single", "pair", "tile", "march", "swap")
 _lib = None
 
 
@@ -88,6 +89,7 @@ def load():
         "mplbhip_iterate_batch": (I, [P, D, I, ctypes.c_longlong, LLP, DP, LLP]),
         "mplbhip_set_batch_restart": (I, [P, D]),
         "mplbhip_launch_shape": (I, [P, IP, IP, IP, LLP]),
+        "mplbhip_step_form": (I, [P, IP, IP]),
         "mplbhip_batch_restarts": (I, [P, IP]),
     }
     for name, (res, args) in sig.items():
@@ -291,6 +293,13 @@ class LatticeCase:
         self._ck(self.lib.mplbhip_launch_shape(self.h, ctypes.byref(f), ctypes.byref(x),
                                                ctypes.byref(h), ctypes.byref(nodes)))
         return f.value, x.value, h.value, nodes.value
+
+    def step_form(self):
+        """(form, steps of one launch) of step(): "single", "pair", "tile",
+        "march" or "swap"."""
+        f, n = ctypes.c_int(), ctypes.c_int()
+        self._ck(self.lib.mplbhip_step_form(self.h, ctypes.byref(f), ctypes.byref(n)))
+        return STEP_FORMS[f.value], n.value
 
     def set_batch_restart(self, factor):
         """Restart, once, a batched instance whose residual climbs above
