@@ -281,6 +281,8 @@ static int upload_blocks(mplbhip_ctx* c) {
     return 0;
 }
 
+static int assign_2d(mplbhip_ctx* c, bool only_active);
+
 static void drop_graphs(mplbhip_ctx* c) {
     for (int i = 0; i < 2; i++) {
         if (c->gexec[i]) (void)hipGraphExecDestroy(c->gexec[i]);
@@ -506,8 +508,8 @@ static int enqueue_step(mplbhip_ctx* c, bool check, bool residual) {
     return 0;
 }
 
-// steps per launch in force (1: single steps); a body force given after
-// prepare turns the forms without one off
+// steps per launch in force (1: single steps); a body force turns the forms
+// without one off
 static int launch_steps(const mplbhip_ctx* c) {
     if (c->swap || c->thermal) return 1;
     if (c->tile) return tile_max_steps(c->tile_side);
@@ -805,8 +807,11 @@ int mplbhip_define_collision(mplbhip_ctx* c, double tau_ref, int force_type,
     c->force_type = force_type;
     c->force_macros = force_macros ? 1 : 0;
     if (c->prepared && c->device >= 0) {
+        HIPCHK(c, hipSetDevice(c->device));
         drop_graphs(c);
-        return upload_blocks(c);
+        if (int rc = upload_blocks(c)) return rc;
+        // a body force may take 2D steps from rows to tiles, or back
+        return assign_2d(c, false);
     }
     return 0;
 }
@@ -2283,6 +2288,8 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
     // steps between checks: 1,000 steps in 2.18 ms with graphs of 4 launches,
     // 2.09 of 8, 2.11 of 16, that is none).
     const int ls = launch_steps(c);
+    if (ls == 1 && nsteps > 0)
+        if (int rc = tune_single(c)) return rc;
     int G = std::max(32, 16 * ls);
     if (const char* e = std::getenv("MPLBHIP_GRAPH_STEPS")) {
         const int g = std::atoi(e);
