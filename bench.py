@@ -3,11 +3,11 @@
 D3Q19, 256^3 nodes, Re = 400, lid speed 0.05 (lattice units), rest state plus
 seeded density noise +-1e-4, populations stored as f - w_i in FP32.
 
-One step = the bulk kernel (fused pull stream + macros + BGK collision over
-the interior nodes) and the boundary kernel (the region programs of the
-block's faces, edges and corners).  Inputs are resident in HBM before the
-timed region.  The roofline figure is that of the bulk kernel, which moves
-(n-2)^3 nodes x 19 populations x (read + write).  Prints one JSON line.
+Two steps (pull stream, walls, macros, BGK collision) take one launch, and a
+run ends with one or two single steps.  Inputs are resident in HBM before the
+timed region.  The roofline figure is that of these launches, which read and
+write n^3 nodes x 19 populations once each; the single-step kernels' own
+figure is beside it.  Prints one JSON line.
 
   python bench.py [--gpus 1] [--steps 2000] [--warmup 50]
 """
@@ -53,6 +53,50 @@ def traffic_from_profiles(name):
         return d.get("traffic_bytes_per_launch")
     except (OSError, ValueError):
         return None
+
+
+KERNELS = {"single": "k_bulk and k_lattice", "pair": "k_pair", "tile": "k_tile", "march": "k_march",
+           "swap": "k_swap_pull"}
+GRAPH_STEPS = 32
+
+
+def launch_plan(form, per, steps):
+    """(launches of several steps, single steps, steps in graph replays) of
+    step(steps) in a form of `per` steps per launch."""
+    if per == 1:
+        return 0, steps, steps // GRAPH_STEPS * GRAPH_STEPS
+    graph = max(GRAPH_STEPS, 16 * per)
+    graph -= graph % per
+    left = max(steps - 1, 0)  # the last step is a single one
+    multi, rest = divmod(left, per)
+    if form == "tile" and rest >= 2:
+        multi, rest = multi + 1, 0
+    return multi, min(steps, 1) + rest, left // graph * graph
+
+
+def roofline(g, q, elem, nodes, steps):
+    """The kernels of `steps` more steps, event-timed launch by launch as
+    step() makes them, against HBM: every launch has to read and to write the
+    lattice once, whether it takes one step or several."""
+    form, per = g.step_form()
+    multi, single, graphed = launch_plan(form, per, steps)
+    _, ms = g.step_timed(steps)
+    moved = 2 * q * elem * nodes
+    achieved = moved * (multi + single) / (ms / 1e3) / 1e9
+    kernel = KERNELS[form]
+    how = ("%d steps in %d launches of %s and %d single steps" % (steps, multi, kernel, single)
+           if multi else "%d single steps" % steps)
+    return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+            "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "kernel": "%s (D%dQ%d)" % (kernel, 2 if q == 9 else 3, q),
+            "steps_per_launch": per, "launches": multi + single,
+            "algorithmic_bytes": moved,
+            "kernel_avg_ms": round(ms / (multi + single), 5),
+            "kernel_ms_per_step": round(ms / steps, 5),
+            "timing": "value: %s, %s; this roofline: the same launches once more, one by one "
+                      "with HIP events around each kernel"
+                      % (how, "%d of them in graph replays" % graphed if graphed
+                         else "launched one by one")}
 
 
 def host_info():
@@ -182,11 +226,7 @@ def bench_lchannel(args):
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
-                     "traffic_source": ("profiles/%s (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE "
-                                        "for this launch shape, scaled by the copy-kernel "
-                                        "calibration; not measured in this run)" % tname)
-                     if traffic else
-                     "no committed counter summary for this launch shape (%s)" % tname,
+                     "traffic_source": traffic_source(tname, traffic),
                      "kernel": "k_bulk (D3Q19, %s, step)" % st,
                      "bulk_nodes_per_launch": bulk_nodes,
                      "launch_shape": {"fold": fold, "xgroup": xgroup, "h2": h2},
@@ -198,6 +238,55 @@ def bench_lchannel(args):
         "wall_s": round(wall, 3),
         "error_vs_fp64": err,
     }
+
+
+def launch_traffic(workload, storage, roof):
+    """(HBM bytes of one launch, where that comes from) by the committed
+    counter summary of a kernel of several steps."""
+    name = "%s_%s_%s_traffic.json" % (roof["kernel"].split()[0], workload, storage)
+    traffic = traffic_from_profiles(name)
+    return traffic, traffic_source(name, traffic)
+
+
+def traffic_source(name, traffic):
+    if traffic:
+        return ("profiles/%s (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE for this launch shape, "
+                "scaled by the copy-kernel calibration; not measured in this run)" % name)
+    return "no committed counter summary for this launch shape (%s)" % name
+
+
+def single_step_roofline(n, st, copy_gbs, steps=100):
+    """The single-step kernels of the same cavity, a run's last ones: bulk and
+    boundary kernel with events around each.  Bytes: 2 Q s for every node that
+    the bulk kernel updates."""
+    before = os.environ.get("MPLBHIP_PAIR")
+    os.environ["MPLBHIP_PAIR"] = "0"
+    try:
+        g = hip.LatticeCase(3, storage=STORE[st], device=0)
+        cases.cavity3d(g, n, re=400.0, ulid=0.05, noise=True)
+    finally:
+        if before is None:
+            del os.environ["MPLBHIP_PAIR"]
+        else:
+            os.environ["MPLBHIP_PAIR"] = before
+    g.step(steps)
+    g.step_timed(steps)
+    ms_bulk, ms_bnd = g.kernel_times()
+    fold, xgroup, h2, bulk_nodes = g.launch_shape()
+    g.close()
+    bulk_bytes = bulk_nodes * 2 * 19 * ELEM[st]
+    achieved = bulk_bytes / (ms_bulk / steps / 1e3) / 1e9
+    name = traffic_profile_name("d3q19_%d" % n, st, fold, xgroup)
+    traffic = traffic_from_profiles(name)
+    return {"achieved": round(achieved, 1), "unit": "GB/s",
+            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "frac_of_copy": round(achieved / copy_gbs, 4),
+            "traffic": traffic, "traffic_source": traffic_source(name, traffic),
+            "kernel": "k_bulk (D3Q19, %s, step)" % st, "algorithmic_bytes": bulk_bytes,
+            "bulk_nodes_per_launch": bulk_nodes,
+            "launch_shape": {"fold": fold, "xgroup": xgroup, "h2": h2},
+            "kernel_avg_ms": round(ms_bulk / steps, 5),
+            "boundary_kernel_avg_ms": round(ms_bnd / steps, 5)}
 
 
 def bench_batch(args):
@@ -213,22 +302,17 @@ def bench_batch(args):
     cases.batched_cavities(g, sizes, res)
     g.step(args.warmup)
     g.sync()
-    # the value: K steps as graph replays (the path iterate_batch runs);
-    # then the kernel split from K more steps with events around each kernel
+    # the value: K steps (the path iterate_batch runs); then the kernels'
+    # times from K more steps with events around each launch
     t0 = time.perf_counter()
     g.step(args.steps)
     g.sync()
     wall = time.perf_counter() - t0
     mlups = nodes * args.steps / wall / 1e6
-    _, ker = g.step_timed(args.steps)
-    b, d = g.kernel_times()
-    fold, xgroup, h2, bulk_nodes = g.launch_shape()
-    achieved = bulk_nodes * 2 * 9 * ELEM[st] / (b / args.steps / 1e3) / 1e9
-    tname = traffic_profile_name("batch%d" % len(sizes), st, fold, xgroup)
-    traffic = traffic_from_profiles(tname)
-    log("bench: batch %.0f MLUPS (wall, graph replays), event-timed kernels %.4f ms/step "
-        "(bulk %.4f = %.0f GB/s, boundary %.4f)"
-        % (mlups, ker / args.steps, b / args.steps, achieved, d / args.steps))
+    roof = roofline(g, 9, ELEM[st], nodes, args.steps)
+    roof["traffic"], roof["traffic_source"] = launch_traffic("batch%d" % len(sizes), st, roof)
+    log("bench: batch %.0f MLUPS (wall), event-timed kernels %.4f ms/step (%s, %.0f GB/s)"
+        % (mlups, roof["kernel_ms_per_step"], roof["kernel"], roof["achieved"]))
     conv = None
     if args.converge:
         t0 = time.perf_counter()
@@ -253,20 +337,8 @@ def bench_batch(args):
         "config": {"workload": "%d D2Q9 lid-driven cavities, N in {64..256}, Re in "
                                "[100,1000], lid 0.05, %s storage" % (len(sizes), st),
                    "nodes": nodes},
-        "kernel_ms_per_step": round(ker / args.steps, 5),
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "traffic_source": ("profiles/%s (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE "
-                                        "for this launch shape, scaled by the copy-kernel "
-                                        "calibration; not measured in this run)" % tname)
-                     if traffic else
-                     "no committed counter summary for this launch shape (%s)" % tname,
-                     "kernel": "k_bulk (D2Q9, %s, step)" % st,
-                     "bulk_nodes_per_launch": bulk_nodes,
-                     "launch_shape": {"fold": fold, "xgroup": xgroup, "h2": h2},
-                     "bulk_ms_per_step": round(b / args.steps, 5)},
-        "timing": "value: K steps of graph replays (the path iterate_batch runs); kernel times: "
-                  "HIP events around every kernel of K more steps launched one by one",
+        "kernel_ms_per_step": roof["kernel_ms_per_step"],
+        "roofline": roof,
         "convergence": conv,
     }
 
@@ -492,40 +564,35 @@ def main():
     if W > 0:
         g.step(W)
     # the timed region: K steps of the production path (mplbhip_step, the
-    # same replays of captured 32-step graphs that Iterate runs)
+    # same launches and graph replays that Iterate runs)
     g.sync()
     t0 = time.perf_counter()
     g.step(K)
     g.sync()
     wall = time.perf_counter() - t0
-    # then K more steps launched one by one with HIP events around each
-    # kernel on the stream it runs on (a captured graph cannot carry
-    # timing events): the kernels' average durations for the roofline
+    # then K more steps with HIP events around each launch (a captured graph
+    # cannot carry timing events): the kernels' durations for the roofline
     g.sync()
     t1 = time.perf_counter()
-    ms_gpu_span, ms_kernel = g.step_timed(K)
+    roof = roofline(g, 19, ELEM[st], n ** 3, K)
     g.sync()
     wall_events = time.perf_counter() - t1
-    ms_bulk, ms_bnd = g.kernel_times()
+    roof["ms_per_step_event_timed"] = round(wall_events / K * 1e3, 5)
     nodes = n ** 3
     mlups = nodes * K / wall / 1e6
     q = 19
-    bulk_s = ms_bulk / K / 1e3
-    # algorithmic bytes per bulk launch: 2 Q s for every node it updates
-    # (the interior, plus the boundary nodes folded into it at fold level
-    # 1 or 2); the interior-only figure is kept beside it
-    fold, xgroup, h2, bulk_nodes = g.launch_shape()
-    bulk_bytes = bulk_nodes * 2 * q * ELEM[st]
-    interior_bytes = (n - 2) ** 3 * 2 * q * ELEM[st]
-    achieved = bulk_bytes / bulk_s / 1e9
-    log("bench: wall %.3f s (graph replays), %.3f s with per-kernel events (gpu span "
-        "%.3f ms), bulk kernel avg %.4f ms (%.0f GB/s), boundary kernel avg %.4f ms, "
-        "%.0f MLUPS" % (wall, wall_events, ms_gpu_span, bulk_s * 1e3, achieved, ms_bnd / K,
-                        mlups))
+    log("bench: wall %.3f s, %.3f s with events around each launch, %s avg %.4f ms "
+        "(%.0f GB/s), %.0f MLUPS" % (wall, wall_events, roof["kernel"], roof["kernel_avg_ms"],
+                                     roof["achieved"], mlups))
 
     copy_bytes = 2 << 30
     copy_ms = hip.copy_probe(copy_bytes, iters=20)
     copy_gbs = 2 * copy_bytes / (copy_ms / 1e3) / 1e9
+    roof["copy_probe_GBs"] = round(copy_gbs, 1)
+    roof["frac_of_copy"] = round(roof["achieved"] / copy_gbs, 4)
+    roof["traffic"], roof["traffic_source"] = launch_traffic("d3q19_%d" % n, st, roof)
+    if roof["steps_per_launch"] > 1:
+        roof["single_step"] = single_step_roofline(n, st, copy_gbs)
 
     err = None
     if not args.no_error and st != "f64":
@@ -552,7 +619,6 @@ def main():
         log("bench: CPU oracle baseline (about %.0f s at %d^3)" % (args.cpu_seconds, n))
         cpu = cpu_baseline(n, args.cpu_seconds)
 
-    tname = traffic_profile_name("d3q19_%d" % n, st, fold, xgroup)
     out = {
         "metric": METRIC,
         "value": round(mlups, 1),
@@ -570,30 +636,7 @@ def main():
                                "%s storage (f - w_i)" % (n, st),
                    "nodes": nodes, "lattice": "D3Q19", "storage": st,
                    "bytes_per_lattice_update": 2 * q * ELEM[st]},
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1),
-                     "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": traffic_from_profiles(tname),
-                     "traffic_source": ("profiles/%s (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE "
-                                        "for this launch shape, scaled by the copy-kernel "
-                                        "calibration; not measured in this run)" % tname)
-                     if traffic_from_profiles(tname) else
-                     "no committed counter summary for this launch shape (%s)" % tname,
-                     "kernel": "k_bulk (D3Q19, %s, step)" % st,
-                     "algorithmic_bytes": bulk_bytes,
-                     "bulk_nodes_per_launch": bulk_nodes,
-                     "launch_shape": {"fold": fold, "xgroup": xgroup, "h2": h2},
-                     "achieved_interior_only": round(interior_bytes / bulk_s / 1e9, 1),
-                     "kernel_avg_ms": round(bulk_s * 1e3, 5),
-                     "boundary_kernel_avg_ms": round(ms_bnd / K, 5),
-                     "step_kernels_avg_ms": round(ms_kernel / K, 5),
-                     "ms_per_step_event_timed": round(wall_events / K * 1e3, 5),
-                     "timing": "value: K steps of the production path (two steps per launch, "
-                               "k_pair, in graph replays); this roofline: the single-step "
-                               "kernels, HIP events around every kernel of K more steps "
-                               "launched one by one on the same streams",
-                     "copy_probe_GBs": round(copy_gbs, 1),
-                     "frac_of_copy": round(achieved / copy_gbs, 4)},
+        "roofline": roof,
         "cpu_baseline": cpu,
     }
     if err is not None:

@@ -152,13 +152,14 @@ int mplbhip_set_accel(mplbhip_ctx* ctx, int block, const double* g);
 /* StreamCollision x nsteps (evolution.cpp:137-193), queued on the
  * context stream and returned once complete. */
 int mplbhip_step(mplbhip_ctx* ctx, int nsteps);
-/* nsteps timed with HIP events on the context stream around each step
- * kernel: ms_total is the wall span, ms_kernel the summed time of the step
- * kernels (bulk and boundary; halo copies excluded) */
+/* mplbhip_step's launches one by one (no captured graphs) with HIP events
+ * around each step kernel: ms_total is the wall span, ms_kernel the summed
+ * time of the step kernels (halo copies excluded) */
 int mplbhip_step_timed(mplbhip_ctx* ctx, int nsteps, double* ms_total,
                        double* ms_kernel);
 /* Diagnostic, no reference counterpart: the bulk-kernel and boundary-kernel
- * shares of the last mplbhip_step_timed call (ms, summed over its steps). */
+ * shares of the last mplbhip_step_timed call (ms, summed over its steps);
+ * launches that are both, or of several steps, are in the bulk share. */
 int mplbhip_kernel_times(mplbhip_ctx* ctx, double* ms_bulk, double* ms_boundary);
 /* Diagnostic, no reference counterpart: the single-step launch shape in force
  * (after its autotuning: the first step, or where several steps share a

@@ -2214,6 +2214,84 @@ static int first_collision(mplbhip_ctx* c) {
     return launch_steps(c) > 1 ? 0 : autotune(c);
 }
 
+// the steps of a launch of several for which `left` of a run's steps are left,
+// 1: a single step is next
+static int next_launch(const mplbhip_ctx* c, int left) {
+    const int ls = launch_steps(c);
+    return left >= (c->tile ? 2 : ls) ? std::min(ls, left) : 1;
+}
+
+// The launches of mplbhip_step (without captured graphs, which cannot carry
+// events), each step kernel between two events on the stream it runs on: a
+// bulk and a boundary kernel each, any other launch as the bulk share.
+static int timed_steps(mplbhip_ctx* c, int nsteps, double* ms_total, double* ms_kernel) {
+    if (launch_steps(c) == 1 && nsteps > 0)
+        if (int rc = tune_single(c)) return rc;
+    std::vector<hipEvent_t> evs(4 * ((size_t)nsteps + 1));
+    for (auto& e : evs) HIPCHK(c, hipEventCreate(&e));
+    std::vector<char> split;  // per launch: a bulk and a boundary kernel
+    auto bracket = [&](auto&& enqueue) -> int {
+        hipEvent_t* ev = &evs[4 * split.size()];
+        split.push_back(0);
+        HIPCHK(c, hipEventRecord(ev[0], c->stream));
+        if (int rc = enqueue()) return rc;
+        HIPCHK(c, hipEventRecord(ev[1], c->stream));
+        return 0;
+    };
+    HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+    int left = nsteps;
+    if (c->swap_pull && nsteps > 0) {
+        if (int rc = bracket([&] { return swap_begin(c, nsteps); })) return rc;
+        for (; left > 1; left--, c->tstep++)
+            if (int rc = bracket([&] { return swap_pass(c, true); })) return rc;
+        if (int rc = bracket([&] { return swap_end(c); })) return rc;
+        left = 0;
+        c->tstep++;
+    }
+    while (left > 0) {
+        const int n = next_launch(c, left - 1);  // the last step is a single one
+        if (n > 1) {
+            if (int rc = bracket([&] { return enqueue_multi(c, n); })) return rc;
+        } else if (c->swap) {
+            if (int rc = bracket([&] { return enqueue_swap_step(c, false, false); })) return rc;
+        } else {
+            if (int rc = fresh_halos(c)) return rc;
+            const KParams kp = base_params(c);
+            if (kp.fused) {
+                if (int rc = bracket([&]() -> int {
+                        HIPCHK(c, launch_lattice(c->lat, c->storage, MODE_STEP, kp, c->stream));
+                        return 0;
+                    }))
+                    return rc;
+            } else {
+                split.push_back(1);
+                if (int rc = launch_step_kernels(c, kp, MODE_STEP, &evs[4 * (split.size() - 1)]))
+                    return rc;
+            }
+            if (int rc = exchange(c, 1 - c->cur)) return rc;
+            c->cur ^= 1;
+        }
+        c->tstep += n;
+        left -= n;
+    }
+    HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+    HIPCHK(c, hipEventSynchronize(c->ev[1]));
+    float ms = 0.f;
+    HIPCHK(c, hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
+    if (ms_total) *ms_total = ms;
+    c->last_bulk_ms = c->last_bnd_ms = 0.0;
+    for (size_t l = 0; l < split.size(); l++) {
+        HIPCHK(c, hipEventElapsedTime(&ms, evs[4 * l], evs[4 * l + 1]));
+        c->last_bulk_ms += ms;
+        if (!split[l]) continue;
+        HIPCHK(c, hipEventElapsedTime(&ms, evs[4 * l + 2], evs[4 * l + 3]));
+        c->last_bnd_ms += ms;
+    }
+    for (auto& e : evs) (void)hipEventDestroy(e);
+    if (ms_kernel) *ms_kernel = c->last_bulk_ms + c->last_bnd_ms;
+    return 0;
+}
+
 // tail: a check step follows, so the last step need not be a single one
 static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
                      double* ms_kernel, bool tail = false) {
@@ -2224,62 +2302,7 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
     c->swap_run = false;
     if (c->tstep == 0)
         if (int rc = first_collision(c)) return rc;
-    double ktot = 0.0;
-    if (timed) {
-        if (nsteps > 0)
-            if (int rc = tune_single(c)) return rc;
-        if (int rc = fresh_halos(c)) return rc;
-        // per-step events bracket the bulk kernel and the boundary kernel,
-        // each on the stream it runs on (the step's own launch structure)
-        std::vector<hipEvent_t> evs(4 * (size_t)nsteps);
-        for (auto& e : evs) HIPCHK(c, hipEventCreate(&e));
-        HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-        for (int s = 0; s < nsteps; s++) {
-            KParams kp = base_params(c);
-            if (c->swap) {
-                // the whole swap step is the bulk share
-                HIPCHK(c, hipEventRecord(evs[4 * s], c->stream));
-                if (int rc = enqueue_swap_step(c, false, false)) return rc;
-                HIPCHK(c, hipEventRecord(evs[4 * s + 1], c->stream));
-                HIPCHK(c, hipEventRecord(evs[4 * s + 2], c->stream));
-                HIPCHK(c, hipEventRecord(evs[4 * s + 3], c->stream));
-                c->tstep++;
-                continue;
-            }
-            if (kp.fused) {
-                // one whole-lattice launch: it is the bulk share
-                HIPCHK(c, hipEventRecord(evs[4 * s], c->stream));
-                HIPCHK(c, launch_lattice(c->lat, c->storage, MODE_STEP, kp, c->stream));
-                HIPCHK(c, hipEventRecord(evs[4 * s + 1], c->stream));
-                HIPCHK(c, hipEventRecord(evs[4 * s + 2], c->stream));
-                HIPCHK(c, hipEventRecord(evs[4 * s + 3], c->stream));
-            } else if (int rc = launch_step_kernels(c, kp, MODE_STEP, &evs[4 * s])) {
-                return rc;
-            }
-            if (int rc = exchange(c, 1 - c->cur)) return rc;
-            c->cur ^= 1;
-            c->tstep++;
-        }
-        HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-        HIPCHK(c, hipEventSynchronize(c->ev[1]));
-        float ms = 0.f;
-        HIPCHK(c, hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
-        if (ms_total) *ms_total = ms;
-        double btot = 0.0;
-        for (int s = 0; s < nsteps; s++) {
-            float k = 0.f, kb = 0.f;
-            HIPCHK(c, hipEventElapsedTime(&k, evs[4 * s], evs[4 * s + 1]));
-            HIPCHK(c, hipEventElapsedTime(&kb, evs[4 * s + 2], evs[4 * s + 3]));
-            ktot += k;
-            btot += kb;
-        }
-        c->last_bulk_ms = ktot;
-        c->last_bnd_ms = btot;
-        ktot += btot;
-        for (auto& e : evs) (void)hipEventDestroy(e);
-        if (ms_kernel) *ms_kernel = ktot;
-        return 0;
-    }
+    if (timed) return timed_steps(c, nsteps, ms_total, ms_kernel);
     // untimed: replay captured graphs of G steps (even, so the parity after
     // a graph of single steps is unchanged; MPLBHIP_GRAPH_STEPS overrides),
     // the remainder launch by launch.  32 steps, or 16 launches of several:
@@ -2316,8 +2339,9 @@ static int run_steps(mplbhip_ctx* c, int nsteps, bool timed, double* ms_total,
             left -= G;
         }
     }
-    while (ls > 1 && left - keep >= (c->tile ? 2 : ls)) {
-        const int n = std::min(ls, left - keep);
+    while (ls > 1) {
+        const int n = next_launch(c, left - keep);
+        if (n == 1) break;
         if (int rc = enqueue_multi(c, n)) return rc;
         c->tstep += n;
         left -= n;
