@@ -123,7 +123,7 @@ enum Mode : int {
 // Two steps in one launch (k_pair): the tiling of one block.  A workgroup
 // owns w x h columns of one range of lz z planes and marches through them;
 // it computes the first of the two steps on its tile plus one node on every
-// side.  nt: threads of the workgroup, at least (w + 2)(h + 2).
+// side (pair_fits: the positions and threads that takes).
 struct PairBlock {
     int32_t start;       // first workgroup of this block
     int32_t w, h, lz;
@@ -134,8 +134,8 @@ struct PairBlock {
 };
 
 // Several steps in one launch of 2D blocks (k_march): one wave's share.  Its
-// lanes form groups of `group` lanes, each over `group` * C columns from x0
-// on; group g marches through the rows of chunk chunk0 + g (rows of them).
+// lanes form groups of `group` lanes, each over `group` columns from x0 on;
+// group g marches through the rows of chunk chunk0 + g (rows of them).
 struct MarchWave {
     int32_t block;
     int32_t x0;      // first column

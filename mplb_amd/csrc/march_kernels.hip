@@ -70,8 +70,8 @@ __device__ __forceinline__ void march_wall(const MPLB_CONST RegionProg* progs,
 // arithmetic; the wall constants come by scalar loads, and the rows that make
 // no result store out of range, since a vector load or a store under a branch
 // would make the wait for the row wait for those too.  us per step, single
-// steps and march (rows 16): FP32 2048^2 56 and 24.8 (K = 7), 256 blocks of 80
-// to 128 rows 92 and 39 (K = 6); FP64 2048^2 112 and 46 (K = 5); FP16 2048^2 34 and 22.8
+// steps and march (rows 16): FP32 2048^2 56 and 24.8 (K = 7), 256 blocks of 64
+// to 256 rows 94 and 37 (K = 7); FP64 2048^2 112 and 46 (K = 5); FP16 2048^2 34 and 22.8
 // (K = 4); FP32 with obstacles, 96 blocks of 128^2, 25.3 and 16.0 (K = 4).
 template <int ST, int K, bool OBST, int W>
 __global__ __launch_bounds__(64, W) void k_march(KParams kp) {

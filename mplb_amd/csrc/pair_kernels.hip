@@ -235,7 +235,7 @@ __device__ __forceinline__ TileNode tile_node(int tid, bool lo, bool hi, int xr,
 // but one plane at either end of its range.  Tile height and width are what
 // the positions in LDS allow: all populations of one to three planes (38
 // values per position in D3Q19), one workgroup per CU.
-// 256^3 FP32: HBM reads 1.47 GB and writes 1.28 GB per two steps, 4.9 TB/s;
+// 256^3 FP32: HBM reads 1.46 GB and writes 1.28 GB per two steps, 4.9 TB/s;
 // 0.445 -> 0.281 ms per step (FP64 0.957 -> 0.595, FP16 0.237 -> 0.214, where
 // the arithmetic of 16 waves per CU bounds it).  160^3 FP64 0.238 -> 0.159,
 // 81 x 67 x 53 FP64 30.6 -> 24.2 us.  What remains above HBM's time is the
