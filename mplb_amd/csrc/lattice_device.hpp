@@ -193,8 +193,9 @@ __device__ __forceinline__ double bit_sel(uint32_t m, int q, double a, double b)
 // sum_in f / den, a parallel population (w rho_w) res, an outgoing one f_opp
 // + (w rho_w) (2 cu).  Every rounding is the reference's: a factor two and an
 // added zero are exact.  The classes are chosen by bit masks, so the code has
-// no branch, and only incoming populations are read, so that no other one,
-// finite or not, has a part in the result.  With a scalar branch per
+// no branch, and only incoming populations are read (the opposite of an
+// outgoing one is incoming, that of a parallel one parallel), so that no other
+// one, finite or not, has a part in the result.  With a scalar branch per
 // population and class an application took some 60 branches and as many
 // dependent scalar loads, which set the pace of every workgroup that waits
 // for its wall lanes.
@@ -202,18 +203,21 @@ template <int D, typename T, typename OP>
 __device__ __forceinline__ void apply_eqm(T* f, const OP& op) {
 #pragma clang fp contract(off)
     constexpr int Q = lq(D);
-    const uint32_t m_in = op.m_in, m_out = op.m_out, m_set = op.m_out | op.m_par;
-    T rin = T(0);
+    const uint32_t m_in = op.m_in, m_set = op.m_out | op.m_par;
+    T rin = T(0), in[Q];
 #pragma unroll
-    for (int q = 0; q < Q; q++) rin += bit_and(f[q], m_in, q);
+    for (int q = 0; q < Q; q++) {
+        in[q] = bit_and(f[q], m_in, q);
+        rin += in[q];
+    }
     const T rw = T(2) * rin / eq_den(op, T(0));
 #pragma unroll
     for (int q = 0; q < Q; q++) {
         const int p = opp(D, q);
         if (p < q) continue;
         const T wr = T(wgt(D, q)) * rw;
-        const T vq = wr * eq_coef(op, q, T(0)) + bit_and(f[p], m_out, q);
-        const T vp = wr * eq_coef(op, p, T(0)) + bit_and(f[q], m_out, p);
+        const T vq = wr * eq_coef(op, q, T(0)) + in[p];
+        const T vp = wr * eq_coef(op, p, T(0)) + in[q];
         f[q] = bit_sel(m_set, q, vq, f[q]);
         if (p != q) f[p] = bit_sel(m_set, p, vp, f[p]);
     }
@@ -227,13 +231,16 @@ __device__ __forceinline__ void apply_eqm(T* f, const OP& op) {
 template <int D, typename OP>
 __device__ __forceinline__ void apply_eqm_dev(float* g, const OP& op) {
     constexpr int Q = lq(D);
-    const uint32_t m_in = op.m_in, m_out = op.m_out, m_par = op.m_par, m_set = m_out | m_par;
-    float rin = op.eq_win;
+    const uint32_t m_in = op.m_in, m_par = op.m_par, m_set = op.m_out | m_par;
+    float rin = op.eq_win, in[Q];
 #pragma unroll
-    for (int q = 0; q < Q; q++) rin += bit_and(g[q], m_in, q);
+    for (int q = 0; q < Q; q++) {
+        in[q] = bit_and(g[q], m_in, q);
+        rin += in[q];
+    }
     const float rw = rin * op.eq_k;
     auto value = [&](int q, int p) {
-        const float b = bit_or(bit_and(g[p], m_out, q), bit_and(-float(wgt(D, q)), m_par, q));
+        const float b = bit_or(in[p], bit_and(-float(wgt(D, q)), m_par, q));
         return __builtin_fmaf(rw, op.eq_c[q], b);
     };
 #pragma unroll
