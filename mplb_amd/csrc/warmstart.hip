@@ -61,13 +61,13 @@ struct ConvTile {
 // pixels staged for a tile of tp pixels: the largest (R + 2)(W0 + 2)
 __host__ __device__ constexpr int conv_max_staged(int tp) { return tp == 256 ? 340 : 204; }
 
-// equal columns of at most 32, or of as many more as an image of few rows
-// leaves pixels for (1 x 100000, 16 to 16 channels: 11.8 us, 22.4 in columns of
-// 32), and as many rows as the tile's pixels and the staged ones allow
-__host__ __device__ inline ConvTile conv_tile(int h, int wd, int tp) {
+// equal columns of at most 32, or (wide) of as many more as an image of few
+// rows leaves pixels for, and as many rows as the tile's pixels and the staged
+// ones allow
+inline ConvTile conv_tile(int h, int wd, int tp, bool wide) {
     ConvTile t;
     int most = 32;
-    if (h < 8) {
+    if (wide && h < 8) {
         const int row = tp / h, fit = conv_max_staged(tp) / (h + 2) - 2;
         const int w = row < fit ? row : fit;
         if (w > most) most = w;
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const
                                                           const float* __restrict__ bias,
                                                           float* __restrict__ out, int n,
                                                           int h, int wd, int cin, int cout,
-                                                          int relu) {
+                                                          int relu, ConvTile T) {
     constexpr int TP = 128 * WM, CG = 32 * WN, NT = 64 * kWaves;
     constexpr bool WIDE = FORM == kFormWide, VEC = FORM == kFormVec;
     using Off = Offset<FORM>;
@@ -153,7 +153,6 @@ __global__ __launch_bounds__(64 * kWaves, WN == 1 ? 3 : 2) void k_conv_fwd(const
     __shared__ __attribute__((aligned(16))) short s_in[conv_max_staged(TP) * kPixStride];
     // A fragments: [tap][8 input channels][co 0 .. CG-1][8]
     __shared__ __attribute__((aligned(16))) short s_w[9 * (kCC / 8) * CG * 8];
-    const ConvTile T = conv_tile(h, wd, TP);
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int row = lane & 31, g = lane >> 5;
@@ -391,11 +390,11 @@ constexpr int kGWaves = 9;
 constexpr int kGPix = 256;   // pixels of dout staged
 constexpr int kGIn = 396;    // and of the input: (RT + 2)(SEG + 2), 4 lines of 64 the most
 
-// positions and lines of a sub-tile
+// positions and lines of a sub-tile, by those of a whole chunk
 struct GradTile {
     int seg, segs, rt;
 };
-__host__ __device__ inline GradTile grad_tile(int lines, int positions) {
+inline GradTile grad_tile(int lines, int positions) {
     GradTile t;
     const int most = lines == 1 ? 128 : lines == 2 ? 96 : 64;
     t.segs = (positions + most - 1) / most;
@@ -445,7 +444,7 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
                                                                 float* __restrict__ partial,
                                                                 float* __restrict__ bpart, int h,
                                                                 int wd, int cin, int cout,
-                                                                int rows) {
+                                                                int rows, GradTile T) {
     constexpr int NT = 64 * kGWaves, NP = NT / 4;
     constexpr bool WIDE = FORM == kFormWide;
     using Off = Offset<FORM>;
@@ -462,7 +461,6 @@ __global__ __launch_bounds__(64 * kGWaves) void k_conv_wgrad(const float* __rest
     // the chunk's lines and their positions, the pixels from one to the next
     const int nl = TURN ? wd : r1 - r0, np = TURN ? r1 - r0 : wd;
     const int ls = TURN ? 1 : wd, ps = TURN ? wd : 1;
-    const GradTile T = grad_tile(nl, np);
     // the chunk's rows of dout, and of the input with one around
     const int ya = r0 > 0 ? r0 - 1 : 0, yb = r1 < h ? r1 + 1 : h;
     const uint32_t xbytes = (uint32_t)(yb - ya) * (uint32_t)wd * (uint32_t)cin * 4u;
@@ -892,9 +890,16 @@ int mplbws_conv3x3_fwd(const float* in, const float* w, const float* bias, float
     // them and 22.6 us, 28.8 with WM = 1; 128 or fewer: the same within 0.3 us)
     const int wn = cout > 32 ? 2 : 1;
     const int64_t groups = (cout + 32 * wn - 1) / (32 * wn);
-    const ConvTile T2 = conv_tile(h, wd, 256);
-    const int wm = (int64_t)n * T2.tiles_x * T2.tiles_y * groups >= 512 ? 2 : 1;
-    const ConvTile T = conv_tile(h, wd, 128 * wm);
+    auto tiles = [&](int tp, bool longer) {
+        const ConvTile t = conv_tile(h, wd, tp, longer);
+        return (int64_t)n * t.tiles_x * t.tiles_y;
+    };
+    // longer tiles for few rows once there are two short ones for every CU (1 x
+    // 100000, 16 to 16 channels: 22.4 us in columns of 32, 11.8; 1 x 4096, 64 to
+    // 64: 10.1, 10.7)
+    const bool longer = tiles(128, false) * groups >= 512;
+    const int wm = tiles(256, longer) * groups >= 512 ? 2 : 1;
+    const ConvTile T = conv_tile(h, wd, 128 * wm, longer);
     const int64_t wgs = (int64_t)n * T.tiles_x * T.tiles_y;
     if (wgs >= ((int64_t)1 << 31)) return MPLBWS_ERR_ARG;
     const dim3 grd((unsigned)wgs, (unsigned)groups), blk(64 * kWaves);
@@ -904,7 +909,7 @@ int mplbws_conv3x3_fwd(const float* in, const float* w, const float* bias, float
 #define X(WM, WN, FORM)                                                                        \
     if (wm == WM && wn == WN && form == FORM)                                                  \
         hipLaunchKernelGGL((k_conv_fwd<WM, WN, FORM>), grd, blk, 0, 0, in, w, bias, out, n, h, \
-                           wd, cin, cout, relu);
+                           wd, cin, cout, relu, T);
     X(2, 2, kFormAny) X(2, 1, kFormAny) X(1, 2, kFormAny) X(1, 1, kFormAny)
     X(2, 2, kFormVec) X(2, 1, kFormVec) X(1, 2, kFormVec) X(1, 1, kFormVec)
     X(2, 2, kFormWide) X(2, 1, kFormWide) X(1, 2, kFormWide) X(1, 1, kFormWide)
@@ -939,13 +944,14 @@ int mplbws_conv3x3_wgrad(const float* in, const float* dout, float* dw, float* d
     float* bp = dbias ? workspace + chunks * cnt : nullptr;
     const dim3 grd((unsigned)((cin + 31) / 32), (unsigned)((cout + 31) / 32), (unsigned)chunks);
     const bool turn = grad_tiles(wd, rows) < grad_tiles(rows, wd);
+    const GradTile T = turn ? grad_tile(wd, rows) : grad_tile(rows, wd);
     const int64_t most = std::max(cin, cout);
     const bool wide = (int64_t)(rows + 2) * wd >= (((int64_t)1 << 30) + most - 1) / most;
     const int form = wide ? kFormWide : vec4(in, dout, cin, cout, 0) ? kFormVec : kFormAny;
 #define X(FORM, TURN)                                                                           \
     if (form == FORM && turn == TURN)                                                           \
         hipLaunchKernelGGL((k_conv_wgrad<FORM, TURN>), grd, dim3(64 * kGWaves), 0, 0, in, dout, \
-                           workspace, bp, h, wd, cin, cout, rows);
+                           workspace, bp, h, wd, cin, cout, rows, T);
     X(kFormAny, false) X(kFormVec, false) X(kFormWide, false)
     X(kFormAny, true) X(kFormVec, true) X(kFormWide, true)
 #undef X
