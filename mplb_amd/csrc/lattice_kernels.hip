@@ -114,7 +114,8 @@ __global__ __launch_bounds__(kTX * kTY) void k_lattice(KParams kp) {
                     const int64_t i = (int64_t)q * B.sq + node;
                     next[i] = prev[i];
                 }
-            } else {
+            }
+            if constexpr (MODE == MODE_MATERIALIZE || MODE == MODE_INIT_FEQ) {
                 if (kp.fhost && !kp.fhost_in) {
                     const int64_t nn = (int64_t)B.n[0] * B.n[1] * B.n[2];
                     const int64_t h = B.fbase + ((int64_t)z * B.n[1] + y) * B.n[0] + x;
